@@ -6,17 +6,22 @@
 //
 // The timeline around each unit (measured with per-wave clock stamps and with copies that skip parts of the
 // work, on MI355X at 192 rows x 2048 keys):
-//   * Workgroup g takes units g, g + G, ...; a unit's SPW steps are unrolled, so every load, store and
-//     wait sits at a fixed point and the compiler's wait counts are exact (no branch joins paths with
-//     different numbers of memory operations in flight). Stores that only some lanes or waves make are
-//     buffer stores whose range check drops the others' (no branch around them either).
-//   * Unit u starts at step u % SPW (its waves take their tiles in the same rotated order). Units whose
+//   * Workgroup g takes units g, g + G, ... (two kv heads, two units a workgroup: the second unit is chosen by
+//     length, partner_row). A unit runs as many steps as its length has (an even number: two tile buffers); up to
+//     SPW steps are unrolled with an exit after every second one, so every load, store and wait sits at a fixed
+//     point and the compiler's wait counts are exact (as loops, a unit's further steps drained every request in
+//     flight at the loop's head: 33.3 against 32.4 us per layer). Stores that only some lanes or waves make are
+//     buffer stores whose range check drops the others' (no branch around them either). 192 rows of 300..2048 keys:
+//     25.1 us per layer with every unit at the full row's 8 steps and the second unit g + G, 22.4 like this; all
+//     rows at 2048 keys 32.4 and 32.2; one row of 385 keys 6.0 and 5.5 (k_decode_unit).
+//   * Unit u starts at a step of its own (first_step; its waves take their tiles in the same rotated order). Units whose
 //     streams all start at the same offset and advance in step meet the same memory channels at the same
 //     time: a plain read of the peak-load bytes in this kernel's pattern took 35.2 us with every unit starting
 //     at key 0 and 33.6-33.8 us with the rotation; the decode itself gained 0.2-0.4 us.
-//   * The inputs of unit i + 1 (q, or its qkv / bias / RoPE-table rows) are requested at unit i's first
-//     step and, fused, rotated at its third, when they have long arrived. The metadata of unit i + 2
-//     follows at unit i's first step. At the transition no wave waits for anything but its next tile.
+//   * Unit i + 1 is chosen and its metadata requested at unit i's second step, its inputs (q, or its qkv / bias /
+//     RoPE-table rows) at the third and, fused, rotated after the fourth, when they have long arrived. At the
+//     transition no wave waits for anything but its next tile. The lengths the choice needs are requested behind
+//     the first tiles (ahead of them, with the choice at the first step, all rows at 2048 keys took 32.5 us).
 //   * The first unit's metadata and qkv / bias rows go out before any tile, its table rows as soon as the
 //     position returns and before the tiles, so q is ready about when the first tiles land.
 //   * A unit's k / v / q writes go out after its last step (at its first step, in the middle of the tile
@@ -58,9 +63,60 @@ struct RowMeta {
 struct RowUnit {
   int row, kh, hi;  // keys [0, hi) of cache row crow are attended
   int crow;
-  int rot;  // the unit's first step (units start at different offsets; see k_decode_rows)
+  int n, rot;  // steps (even), and the first one (units start at different offsets; see k_decode_rows)
   rsrc_t kr, vr;
 };
+
+// Steps of a unit of `keys` keys: 4 tiles of 64 keys each, rounded up to an even count (two tile buffers), at
+// least `least`.
+__device__ __forceinline__ int steps_of(int keys, int least) {
+  const int n = (keys + 64 * kRowsNW - 1) / (64 * kRowsNW);
+  return max((n + 1) & ~1, least);
+}
+
+// The first step of a unit in workgroup g: one step on from a workgroup to the next, within a full row's steps (at
+// most 8, as far as the lengths of a 4096-position cache reach in ordinary use: with 16, every second workgroup
+// started at step 0 at 128..2048 keys, 14.1 us per layer at 64 rows against 13.05); step 0 where the unit has no
+// such step. The live tiles come in the same cyclic order whether n counts the full row's steps or only the unit's
+// own, so the sums are the same bits (the unfused launch requests its first tiles before it knows the length).
+__device__ __forceinline__ int first_step(int g, int cache_len, int n) {
+  const int nf = min(steps_of(cache_len, 2), 8);
+  int r = g & 7;
+  r = nf == 6 ? (r >= 6 ? r - 6 : r) : r & (nf - 1);
+  return r < n ? r : 0;
+}
+
+// The partner of row r of the first h <= 128 rows among the next h: the row whose length has the opposite rank
+// there (the longest of one half with the shortest of the other, ...). Equal lengths rank in row order in the
+// first half and in reverse order in the second, so where every length is the same the partner is row h + r. A
+// bijection of the halves, the same in every wave that asks. a[k], c[k]: the lengths of rows 64 k + lane and
+// h + 64 k + lane, clamped to 0..top (-1 past h). Ranks by ballots; the row at a rank by a search over the values.
+__device__ __forceinline__ int partner_row(const int (&a)[2], const int (&c)[2], int r, int h, int top, int lane) {
+  const int vr = __builtin_amdgcn_readlane(r < 64 ? a[0] : a[1], r & 63);
+  if (!__ballot((a[0] >= 0 && a[0] != vr) || (a[1] >= 0 && a[1] != vr) || (c[0] >= 0 && c[0] != vr) ||
+                (c[1] >= 0 && c[1] != vr)))
+    return h + r;
+  int t = h - 1;  // the rank to find: h - 1 - the rows ranked before r
+#pragma unroll
+  for (int k = 0; k < 2; ++k) t -= __popcll(__ballot(a[k] > vr || (a[k] == vr && 64 * k + lane < r)));
+  int lo = 0, hi = top;  // the largest x with more than t rows of length >= x
+  while (lo < hi) {
+    const int x = (lo + hi + 1) >> 1;
+    if (__popcll(__ballot(c[0] >= x)) + __popcll(__ballot(c[1] >= x)) > t)
+      lo = x;
+    else
+      hi = x - 1;
+  }
+  const uint64_t e0 = __ballot(c[0] == lo), e1 = __ballot(c[1] == lo);
+  const int n0 = __popcll(e0), n1 = __popcll(e1);
+  // t - (rows of greater length): the place among the n0 + n1 rows of this length, from the end
+  const int at = n0 + n1 - 1 - (t - __popcll(__ballot(c[0] > lo)) - __popcll(__ballot(c[1] > lo)));
+  const bool second = at >= n0;
+  const uint64_t e = second ? e1 : e0;
+  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(e >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e, 0));
+  const uint64_t hit = __ballot(((e >> lane) & 1) != 0 && before == (second ? at - n0 : at));
+  return h + (second ? 64 : 0) + (hit ? __builtin_ctzll(hit) : 0);
+}
 
 }  // namespace
 
@@ -134,7 +190,6 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
   // layer slower, the deeper queues costing more than they hide)
   constexpr int D = 2;
   warm_kernargs<232>();  // the explicit arguments above span 0x00-0xe7
-  static_assert(SPW % D == 0 && SPW >= 4, "steps per unit");
   // K and V tiles of the two pipeline buffers (each read waits for its tile's DMA with a counted vmcnt)
   __shared__ __attribute__((aligned(16))) uint16_t kb0[NW * kVTile];
   __shared__ __attribute__((aligned(16))) uint16_t kb1[NW * kVTile];
@@ -164,32 +219,47 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
   const rsrc_t map_r = make_rsrc(rowmap, rowmap ? (uint32_t)b * 4u : 0u);
   const rsrc_t pos_r = make_rsrc(si.pos, FUSED ? (uint32_t)b * 4u : 0u);
   const rsrc_t slot_r = make_rsrc(si.slot, FUSED ? (uint32_t)b * 4u : 0u);
-  auto unit_of = [&](int i) { return (int)blockIdx.x + i * G; };
+  // Two units per workgroup over two kv heads (the peak load): workgroups 0 .. 2 h - 1 take the units of the first
+  // h = b / 2 rows, then the same head of the row's partner in the second half, so that every workgroup streams
+  // about the same number of keys; the last workgroup of an odd b takes both heads of the last row
+  const bool pairs = nkv == 2 && G == b && b <= 256;
+  const int half = b >> 1;
   // wave w: tiles w, w + NW, ... of the unit, starting at step rot
-  auto tile_of = [&](int rot, int j) { return w + NW * ((j + rot) & (SPW - 1)); };
-  auto row_of = [&](int i) { return unit_of(i) / nkv; };
-  auto meta_load = [&](int i) {
-    const bool live = i < nmine;
-    const uint32_t o = (uint32_t)(live ? row_of(i) : 0) * 4u;
-    const uint32_t dead = live ? 0u : kOOR;  // past the range: reads 0 without memory traffic
-    RowMeta m;
-    m.craw = bld4(map_r, o + dead);  // without a row map an empty range (no branch around the load)
-    m.lraw = bld4(lens_r, o + dead);
-    m.praw = FUSED ? bld4(pos_r, o + dead) : 0;
-    m.sraw = FUSED ? bld4(slot_r, o + dead) : 0;
-    return m;
+  auto tile_of = [&](const RowUnit &un, int j) {
+    const int s = j + un.rot;
+    return w + NW * (s < un.n ? s : s - un.n);
   };
-  // exact = false: the range is the whole cache row (the length is not waited for; hi is set later)
-  auto resolve = [&](int i, const RowMeta &m, RowUnit &un, bool exact) {
-    const int u = unit_of(i);
+  auto set_unit = [&](int i, int partner, RowUnit &un) {
+    const int u = (int)blockIdx.x + i * G;
     un.row = u / nkv;
     un.kh = u - un.row * nkv;
-    un.rot = u & (SPW - 1);
+    if (pairs && (int)blockIdx.x >= 2 * half) {
+      un.row = b - 1;
+      un.kh = i;
+    } else if (pairs && i > 0) {
+      un.row = partner;
+      un.kh = (int)blockIdx.x & 1;
+    }
+  };
+  auto meta_load = [&](int row) {
+    const uint32_t o = (uint32_t)row * 4u;
+    RowMeta m;
+    m.craw = bld4(map_r, o);  // without a row map an empty range (no branch around the load)
+    m.lraw = bld4(lens_r, o);
+    m.praw = FUSED ? bld4(pos_r, o) : 0;
+    m.sraw = FUSED ? bld4(slot_r, o) : 0;
+    return m;
+  };
+  // exact = false: the range is the whole cache row (the length is not waited for; hi is set later). least: the
+  // fewest steps (a unit that is followed by another takes 4: its first steps carry the next unit's requests)
+  auto resolve = [&](const RowMeta &m, RowUnit &un, bool exact, int least) {
     int crow = un.row;
     if (rowmap) crow = __builtin_amdgcn_readfirstlane(m.craw);  // waits for the row map only when there is one
-    const bool ok = i < nmine && crow >= 0 && crow < cache_rows;
+    const bool ok = crow >= 0 && crow < cache_rows;
     un.crow = ok ? crow : -1;
     un.hi = (ok && exact) ? min(max(__builtin_amdgcn_readfirstlane(m.lraw), 0), cache_len) : 0;
+    un.n = steps_of(exact ? un.hi : cache_len, least);
+    un.rot = first_step((int)blockIdx.x, cache_len, un.n);
     const int64_t cb = (int64_t)(ok ? crow : 0) * s_kb + (int64_t)un.kh * s_kh;
     const uint32_t bound = ok ? (uint32_t)(exact ? un.hi : cache_len) * kRow : 0u;
     un.kr = make_rsrc_wave(kc + cb, bound);
@@ -306,17 +376,17 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
   };
 
   // ---- steps: compute tile j of the current unit from buffer j % D, then request into it tile j + D of the
-  // unit, or tile j + D - SPW of the next (one load sequence, sources selected) ----
+  // unit, or the next unit's first tiles (one load sequence, sources selected) ----
   static_assert(D == 2, "wait counts assume one tile requested between a tile and its reads");
   // K(j+2) goes out as soon as tile j's K operands are in registers and V(j+2) after its P.V operand reads
   // (refilling each buffer at once, as one load sequence after the step, measured 0.2 us per layer slower at
   // the peak load, fused). Issued after V(j) when its reads wait: K(j+1), V(j+1) (unless `tail`) and K(j+2)
   // (when reloading); after K(j): V(j), then K(j+1), V(j+1) (unless `tail`).
   auto step = [&](uint16_t *xk, uint16_t *xv, int j, bool reload, bool tail) __attribute__((always_inline)) {
-    const int t0 = 64 * tile_of(cur.rot, j);
-    const bool in_cur = j + D < SPW;
+    const int t0 = 64 * tile_of(cur, j);
+    const bool in_cur = j + D < cur.n;
     const rsrc_t kr = in_cur ? cur.kr : nxt.kr, vr = in_cur ? cur.vr : nxt.vr;
-    const int tt = in_cur ? tile_of(cur.rot, j + D) : tile_of(nxt.rot, j + D - SPW);
+    const int tt = in_cur ? tile_of(cur, j + D) : tile_of(nxt, j + D - cur.n);
     KTile X[1];
     if (t0 < cur.hi) {
       if (tail)
@@ -335,29 +405,26 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
     }
     if (reload) load_v_lds(xv, vr, (uint32_t)(64 * tt), tl);
   };
-  auto step_k = [&](int j, bool reload, bool tail) __attribute__((always_inline)) {
-    step(kbw[j & 1], vbw[j & 1], j, reload, tail);
+  auto step_k = [&](int par, int j, bool reload, bool tail) __attribute__((always_inline)) {
+    step(kbw[par], vbw[par], j, reload, tail);
   };
   auto first_load = [&](int j) __attribute__((always_inline)) {
-    load_tile_kv(kbw[j & 1], vbw[j & 1], cur.kr, cur.vr, (uint32_t)(64 * tile_of(cur.rot, j)), tl, kl);
+    load_tile_kv(kbw[j & 1], vbw[j & 1], cur.kr, cur.vr, (uint32_t)(64 * tile_of(cur, j)), tl, kl);
   };
-  constexpr int kRopeStep = D < SPW - 1 ? D : SPW - 1;  // the next unit's inputs have arrived by then
 
-  // ---- prologue: unit 0's metadata and q inputs go out before its first tile; unit 1's metadata with them ----
-  RowMeta m0 = meta_load(0);
-  RowMeta mn = meta_load(1);
+  // ---- prologue: unit 0's metadata and q inputs go out before its first tile; the lengths with them ----
+  set_unit(0, 0, cur);
+  RowMeta m0 = meta_load(cur.row), mn;
+  const int least0 = nmine > 1 ? 4 : 2;
   {
-    RowUnit u0;
-    u0.row = row_of(0);
-    u0.kh = unit_of(0) - u0.row * nkv;
     QkvRaw r0;
     if (FUSED) {
       // the table rows go out as soon as the position is in, ahead of every tile (their data would return
       // behind the tiles' otherwise: measured slower with the first tile, or all, requested before the
       // position, and slower again with the table rows read through the scalar cache); the range is exact
-      load_xb(u0, true, r0);
+      load_xb(cur, true, r0);
       load_tab(true, __builtin_amdgcn_readfirstlane(m0.praw), r0);
-      resolve(0, m0, cur, true);
+      resolve(m0, cur, true, least0);
       first_load(0);
       // unit 0's rotation, once its table rows are in
       rope_unit(cur, true, __builtin_amdgcn_readfirstlane(m0.praw), __builtin_amdgcn_readfirstlane(m0.sraw), r0, qc0,
@@ -365,23 +432,49 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
 #pragma unroll
       for (int j = 1; j < D; ++j) first_load(j);
     } else {
-      // unfused: the first tiles go out over the whole cache row before the length returns; the range is
-      // narrowed after them
-      load_q(u0, true, qc0, qc1);
-      resolve(0, m0, cur, false);
+      // unfused: the first tiles go out over the whole cache row before the length returns (as many steps as the
+      // row could need); the range is narrowed after them
+      load_q(cur, true, qc0, qc1);
+      resolve(m0, cur, false, least0);
 #pragma unroll
       for (int j = 0; j < D; ++j) first_load(j);
-      resolve(0, m0, cur, true);
+      const int n = cur.n, rot = cur.rot;
+      resolve(m0, cur, true, least0);
+      cur.n = n;
+      cur.rot = rot;
     }
+  }
+
+  // pairs: the lengths of rows 64 k + lane of each half, behind the first tiles (the partner is needed at step 1)
+  int la[2], lc[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    la[k] = bld4(lens_r, pairs ? (uint32_t)(64 * k + lane) * 4u : kOOR);
+    lc[k] = bld4(lens_r, pairs ? (uint32_t)(half + 64 * k + lane) * 4u : kOOR);
   }
 
   // ---- units 0 .. nmine - 2: every step requests D tiles ahead, across into the next unit ----
   for (int i = 0; i < nmine - 1; ++i) {
+    const int least = i + 2 < nmine ? 4 : 2;
+    // the first four steps carry the next unit's preparation: its row and metadata before step 1, its tile
+    // sources and inputs before step 2, its rotation after step 3 (every load long there by then)
 #pragma unroll
-    for (int j = 0; j < SPW; ++j) {
-      if (j == 0) {
-        // unit i + 1: its tile sources and inputs; unit i + 2's metadata
-        resolve(i + 1, mn, nxt, true);
+    for (int j = 0; j < 4; ++j) {
+      if (j == 1) {
+        int partner = 0;
+        if (pairs && (int)blockIdx.x < 2 * half) {
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            la[k] = 64 * k + lane < half ? min(max(la[k], 0), cache_len) : -1;
+            lc[k] = 64 * k + lane < half ? min(max(lc[k], 0), cache_len) : -1;
+          }
+          partner = partner_row(la, lc, (int)blockIdx.x >> 1, half, cache_len, lane);
+        }
+        set_unit(i + 1, partner, nxt);
+        mn = meta_load(nxt.row);
+      }
+      if (j == 2) {
+        resolve(mn, nxt, true, least);
         if (FUSED) {
           mcur_p = __builtin_amdgcn_readfirstlane(mn.praw);
           mcur_s = __builtin_amdgcn_readfirstlane(mn.sraw);
@@ -390,10 +483,15 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
         } else {
           load_q(nxt, true, qn0, qn1);
         }
-        mn = meta_load(i + 2);
       }
-      step_k(j, true, false);
-      if (FUSED && j == kRopeStep) rope_unit(nxt, true, mcur_p, mcur_s, rn, qn0, qn1, ptn, sdn);
+      step_k(j & 1, j, true, false);
+      if (FUSED && j == 3) rope_unit(nxt, true, mcur_p, mcur_s, rn, qn0, qn1, ptn, sdn);
+    }
+#pragma unroll
+    for (int j = 4; j < SPW; j += 2) {
+      if (j >= cur.n) break;
+      step_k(0, j, true, false);
+      step_k(1, j + 1, true, false);
     }
     // the unit's k / v / q go out after its last step (stored at its first step they cost ~0.45 us per layer at
     // the peak load); no row of the launch reads them back
@@ -409,7 +507,13 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
   }
   // ---- the last unit: no request past its last tile ----
 #pragma unroll
-  for (int j = 0; j < SPW; ++j) step_k(j, j + D < SPW, j + 1 == SPW);
+  for (int j = 0; j < SPW - 2; j += 2) {
+    if (j >= cur.n - 2) break;
+    step_k(0, j, true, false);
+    step_k(1, j + 1, true, false);
+  }
+  step_k(0, cur.n - 2, false, false);
+  step_k(1, cur.n - 1, false, true);
   if (FUSED) rope_store(ptc, sdc);
   finish(cur);
   // tiles past a unit's length are requested but not read: let every DMA land before the wave ends
@@ -433,7 +537,6 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
   constexpr int NW = kRowsNW;
   constexpr int D = 2;  // tiles in flight per wave
   warm_kernargs<232>();
-  static_assert(SPW % D == 0 && SPW >= 4, "steps per unit");
   __shared__ __attribute__((aligned(16))) uint16_t kb0[NW * kVTile];
   __shared__ __attribute__((aligned(16))) uint16_t kb1[NW * kVTile];
   __shared__ __attribute__((aligned(16))) uint16_t vb0[NW * kVTile];
@@ -463,10 +566,11 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
   const int praw = FUSED ? bld4(pos_r, mo) : 0;
   const int sraw = FUSED ? bld4(slot_r, mo) : 0;
 
-  int crow = -1, hi = 0;
+  int crow = -1, hi = 0, n = 2, rot = 0;
   rsrc_t kr, vr;
-  // exact = false: the range is the whole cache row (the length is not waited for; hi is set later)
-  auto resolve = [&](bool exact) {
+  // exact = false: the range is the whole cache row (the length is not waited for; hi is set later). first: the
+  // steps are counted from the range
+  auto resolve = [&](bool exact, bool first) {
     int c = row;
     if (rowmap) c = __builtin_amdgcn_readfirstlane(craw);
     const bool ok = c >= 0 && c < cache_rows;
@@ -476,10 +580,16 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
     const uint32_t bound = ok ? (uint32_t)(exact ? hi : cache_len) * kRow : 0u;
     kr = make_rsrc_wave(kc + cb, bound);
     vr = make_rsrc_wave(vc + cb, bound);
+    if (first) {
+      n = steps_of(exact ? hi : cache_len, 2);
+      rot = first_step(u, cache_len, n);
+    }
   };
-  // wave w: tiles w, w + NW, ... of the unit, starting at step u % SPW (as k_decode_rows)
-  const int rot = u & (SPW - 1);
-  auto tile_of = [&](int j) { return w + NW * ((j + rot) & (SPW - 1)); };
+  // wave w: tiles w, w + NW, ... of the unit, starting at step rot (as k_decode_rows)
+  auto tile_of = [&](int j) {
+    const int s = j + rot;
+    return w + NW * (s < n ? s : s - n);
+  };
   auto first_load = [&](int j) __attribute__((always_inline)) {
     load_tile_kv(kbw[j & 1], vbw[j & 1], kr, vr, (uint32_t)(64 * tile_of(j)), tl, kl);
   };
@@ -512,7 +622,7 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
     r.cs[1] = bld16(cr, og + 64u);
     r.sn[0] = bld16(sr, og);
     r.sn[1] = bld16(sr, og + 64u);
-    resolve(true);
+    resolve(true, true);
     first_load(0);
     // the rotation (rope.h arithmetic), once the table rows are in
     const int srow = __builtin_amdgcn_readfirstlane(sraw);
@@ -552,21 +662,21 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
     const uint32_t qo = (uint32_t)(tl.r16 * s_qh * 2) + 16u * tl.g;
     q0 = bld16(qr, qo);
     q1 = bld16(qr, qo + 64u);
-    resolve(false);
+    resolve(false, true);
 #pragma unroll
     for (int j = 0; j < D; ++j) first_load(j);
-    resolve(true);
+    resolve(true, false);
   }
 
   SoftmaxState S;
   S.reset();
   // tile j + 1 was requested after tile j, except for the last (wait counts as in k_decode_rows)
   static_assert(D == 2, "wait counts assume one tile requested after the one read");
-  auto step = [&](uint16_t *xk, uint16_t *xv, int j) __attribute__((always_inline)) {
+  auto step = [&](uint16_t *xk, uint16_t *xv, int j, bool reload, bool tail) __attribute__((always_inline)) {
     const int t0 = 64 * tile_of(j);
     if (t0 < hi) {
       KTile X[1];
-      if (j + 1 == SPW) {
+      if (tail) {
         read_k_tile<0>(X[0], xk, kl);
         compute_step<1, 0, FUSED>(X, xv, t0, hi, q0, q1, sl2, S, tl, lane, &pt);
       } else {
@@ -574,10 +684,16 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
         compute_step<1, 16, FUSED>(X, xv, t0, hi, q0, q1, sl2, S, tl, lane, &pt);
       }
     }
-    if (j + D < SPW) load_tile_kv(xk, xv, kr, vr, (uint32_t)(64 * tile_of(j + D)), tl, kl);
+    if (reload) load_tile_kv(xk, xv, kr, vr, (uint32_t)(64 * tile_of(j + D)), tl, kl);
   };
 #pragma unroll
-  for (int j = 0; j < SPW; ++j) step(kbw[j & 1], vbw[j & 1], j);
+  for (int j = 0; j < SPW - 2; j += 2) {
+    if (j >= n - 2) break;
+    step(kbw[0], vbw[0], j, true, false);
+    step(kbw[1], vbw[1], j + 1, true, false);
+  }
+  step(kbw[0], vbw[0], n - 2, false, false);
+  step(kbw[1], vbw[1], n - 1, false, true);
   if (FUSED) {  // the unit's k / v / q, after its last step (as k_decode_rows)
     bst16(skr, sko, pt.lo);
     bst16(skr, sko + 64u, pt.hi);

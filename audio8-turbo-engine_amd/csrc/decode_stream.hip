@@ -572,10 +572,13 @@ extern "C" int a8_store_decode_stream(const void *qkv, int64_t s_qkv, const void
 // compute units (k_decode_rows). Measured on MI355X at KV 2048, fused store + decode, us per layer: 128 units
 // (64 rows) 16.6 one per workgroup against 17.9 for the split kernel; 256 units 24.9 against 30.9 for two per
 // workgroup on 128; 288 units 31.5 two per workgroup against 35.9 one per workgroup (32 compute units then
-// hold two); 384 units (C3) 36.2-36.6 two per workgroup against 39.0 one per workgroup. Beyond that, and for
-// other row lengths: a workgroup target of 3/4 of the compute units, chunks per unit only as many as needed to
-// reach it (long rows of few units), and a grid that divides the chunk count evenly. The workspace caps the
-// chunk count per unit.
+// hold two); 384 units (C3) 36.2-36.6 two per workgroup against 39.0 one per workgroup. Rows of up to 64 tiles
+// (a 4096-position cache) do from 5/8 of the compute units: at 200 units of 128..2048 keys 14.6 one per workgroup
+// against 21.0 two per workgroup on 100, at 160 units 14.5 against 15.5 for the split kernel (500..4096 keys: 23.9
+// against 24.4), but at 128 units of 500..4096 keys 22.8 against 20.2, the longest row being one workgroup's.
+// Beyond that, and for other row lengths: a workgroup target of 3/4 of the compute units, chunks per unit only as
+// many as needed to reach it (long rows of few units), and a grid that divides the chunk count evenly. The
+// workspace caps the chunk count per unit.
 extern "C" int a8_decode_choose_stream(int b, int nkv, int cache_len, int64_t cap_row_splits, int n_cu,
                                        int *waves_out, int *tpw_out, int *grid_out) {
   using namespace a8;
@@ -584,7 +587,8 @@ extern "C" int a8_decode_choose_stream(int b, int nkv, int cache_len, int64_t ca
   const int64_t tiles = cache_len > 0 ? (cache_len + 63) / 64 : 1;
   const int nw = tiles >= 8 ? 4 : tiles >= 4 ? 2 : 1;
   const int64_t units = (int64_t)b * nkv;
-  if (nw == 4 && tiles <= 32 && 2 * units >= n_cu && units <= 2 * (int64_t)n_cu) {
+  if (nw == 4 && tiles <= 64 && (tiles <= 32 ? 2 * units >= n_cu : 8 * units >= 5 * (int64_t)n_cu) &&
+      units <= 2 * (int64_t)n_cu) {
     *waves_out = 4;
     *tpw_out = (int)((tiles + 3) / 4);
     *grid_out = (int)(units <= n_cu ? units : (units + 1) / 2);

@@ -143,7 +143,7 @@ class DecodeAttention:
       mode "auto" (default): "stream" when the rows are whole units (row, kv head) of 1024+ keys that
         either give every workgroup of the grid two of them -- the peak-load shape -- or, one per
         workgroup, number at least half the compute units (tick buckets of 64-128 slots at KV 2048); for
-        the fused store + decode (store_and_attend) also when rows are short (cache_len <= 512: one
+        the fused store + decode (store_and_attend) also when rows are short (cache_len <= 1024: one
         workgroup per (row, kv head) holds the whole row, so the store, the decode and the merge take
         one launch); else "split"."""
 
@@ -217,7 +217,10 @@ class DecodeAttention:
         self._shapes[key] = (grid.value,)
         return self._shapes[key]
 
-    SHORT_ROWS = 512  # fused calls: rows of at most this many cache positions take one workgroup each
+    # fused calls: rows of at most this many cache positions take one workgroup each. At 1024 positions (lengths up to
+    # the cache) one launch took 4.8 / 7.4 / 7.9 us at 1 / 8 / 32 rows against 8.1 / 8.9 / 9.6 for split + combine; at
+    # 2048 the long rows turn it round (16 rows of up to 1400 keys: 9.4 against 8.9)
+    SHORT_ROWS = 1024
 
     def short_rows_shape(self, b: int, cache_len: int):
         """Stream mode for short rows: one workgroup per (row, kv head) holding the whole row (up to 4
