@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liba8attn.so")
 SOURCES = ["capi.hip", "store.hip", "decode.hip", "decode_stream.hip", "decode_rows.hip", "decode_flat.hip", "prefill.hip",
            "prefill128.hip", "attn_cols.hip",
-           "prefix_copy.hip", "layer_ops.hip", "gemm.hip", "decode_f32q.hip", "conv.hip"]
+           "prefix_copy.hip", "layer_ops.hip", "gemm.hip", "decode_f32q.hip", "conv.hip", "conv_tile.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -30,46 +30,10 @@
 //     order by a finishing kernel, so results do not depend on timing.
 // The snake's sine runs on the hardware sine unit after an exact reduction to one period.
 // snake_cat: one lane per 8 channels of one output row, 16-byte loads and stores.
-#include "a8_common.h"
+#include "conv_tile.h"
+#include "fp16_ops.h"
 
 namespace a8 {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ f32x4 mfma16x16x32_f16(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                 0);
-}
-// fp16 word <-> fp32 (exact), two fp32 -> one dword of two fp16 (round to nearest even)
-__device__ __forceinline__ float h_lo(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[0]; }
-__device__ __forceinline__ float h_hi(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[1]; }
-__device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi});
-}
-// sin(x) on the hardware sine (v_sin_f32 takes revolutions): x / 2 pi reduced to [-1/2, 1/2] by its nearest
-// integer, so the unit sees its most accurate range; absolute error ~1e-6 for the snake's |a x| < 100, far
-// below the fp16 rounding of the result
-__device__ __forceinline__ float sin_hw(float x) {
-  float r = x * 0.15915494309189535f;
-  r -= __builtin_rintf(r);
-  return __builtin_amdgcn_sinf(r);
-}
-__device__ __forceinline__ u32x2 ld8(const void *p) { return *reinterpret_cast<const u32x2 *>(p); }
-// the snake x + ib sin(a x)^2 on 8 channels (fp32, one rounding to fp16). No contraction: left free, the compiler
-// fuses the last add and the fp16 conversion into one v_fma_mix at some call sites and not at others (one
-// rounding against two), and the same row would get different bits in snake_cat, the conv loads and the state.
-__device__ __forceinline__ u32x4 snake8(u32x4 v, const float *a, const float *ib) {
-#pragma clang fp contract(off)
-  u32x4 o;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float x0 = h_lo(v[j]), x1 = h_hi(v[j]);
-    const float s0 = sin_hw(x0 * a[2 * j]), s1 = sin_hw(x1 * a[2 * j + 1]);
-    o[j] = pack_f16x2(x0 + ib[2 * j] * s0 * s0, x1 + ib[2 * j + 1] * s1 * s1);
-  }
-  return o;
-}
 
 constexpr int kSnakeMaxC = 1024;  // input channels a conv with the snake on its loads may have
 
@@ -606,6 +570,17 @@ static ConvPlan conv_plan(int64_t M, int Cin, int Cout, int taps, int ph, bool a
   return pl;
 }
 
+// k_conv_fin over the partials of `ksplit` shares, rows of NP floats.
+static int launch_fin(const float *part, int64_t NP, int ksplit, const void *bias, const void *res, int64_t s_rb,
+                      int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, int64_t M, int TR, int Cout, int ph,
+                      hipStream_t stream) {
+  const int64_t threads = (int64_t)ph * M * ((Cout + 3) / 4);
+  hipLaunchKernelGGL(k_conv_fin, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, part, NP, ksplit,
+                     (const uint16_t *)bias, (const uint16_t *)res, s_rb, s_rt, (uint16_t *)y, s_yb, s_yt, (int)M, TR,
+                     Cout, ph);
+  return (int)hipGetLastError();
+}
+
 }  // namespace a8
 
 extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void *w, int64_t s_wp, int64_t s_wt,
@@ -645,6 +620,26 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
   ConvPlan pl = conv_plan(M, Cin, Cout, taps, ph);
   if (pl.ksplit > 1 && (!ws || ws_bytes < pl.ws_bytes)) pl = conv_plan(M, Cin, Cout, taps, ph, false);  // one pass
   if (pl.ksplit > 1 && !al16(ws)) return set_error(A8_EALIGN, "conv_cl: workspace must be 16-byte aligned");
+  // the tile kernel where its preconditions hold: batch rows back to back, 16-byte stores, no snake on the load
+  if (!snake_a && (B == 1 || s_xb == (int64_t)Tin * s_xt) && s_xt >= Cin && s_xt <= 65536 && al16(y) &&
+      !((s_yb | s_yt) & 7) && (!res || (al16(res) && !((s_rb | s_rt) & 7))) &&
+      !(reinterpret_cast<uintptr_t>(bias) & 7u)) {
+    ConvTilePlan tp = conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, ph, false, true);
+    if (tp.ksplit > 1 && (!ws || !al16(ws) || ws_bytes < tp.ws_bytes))
+      tp = conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, ph, false, false);
+    if (tp.xkb) {
+      ConvTileArgs a{};
+      a.x = (const uint16_t *)x, a.s_xt = s_xt, a.w = (const uint16_t *)w, a.s_wp = s_wp, a.s_wt = s_wt, a.s_wc = s_wc;
+      a.bias = (const uint16_t *)bias, a.res = (const uint16_t *)res, a.s_rb = s_rb, a.s_rt = s_rt;
+      a.y = (uint16_t *)y, a.s_yb = s_yb, a.s_yt = s_yt, a.M = (int)M, a.TR = TR, a.Tin = Tin, a.Cin = Cin;
+      a.Cout = Cout, a.taps = taps, a.dil = dil, a.ph = ph, a.part = tp.ksplit > 1 ? (float *)ws : nullptr;
+      a.ksplit = tp.ksplit, a.x_span = (uint32_t)x_span, a.w_span = (uint32_t)w_span;
+      const int e = conv_tile_launch(tp, a, false, (hipStream_t)stream);
+      if (e || tp.ksplit == 1) return e;
+      return launch_fin((const float *)ws, Cout, tp.ksplit, bias, res, s_rb, s_rt, y, s_yb, s_yt, M, TR, Cout, ph,
+                        (hipStream_t)stream);
+    }
+  }
   const int NT = pl.NT, WM = pl.WM;
   float *part = pl.ksplit > 1 ? (float *)ws : nullptr;
   const dim3 grid((unsigned)((M + 64 * WM - 1) / (64 * WM)), (unsigned)pl.ntiles, (unsigned)(ph * pl.ksplit));
@@ -708,15 +703,10 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
 #undef A8_CONV_NT_NARROW
 #undef A8_CONV_NT_NO16
 #undef A8_CONV_ARGS
-  if (part) {
-    const hipError_t e = hipGetLastError();  // the finish would sum a workspace the main launch never wrote
-    if (e != hipSuccess) return (int)e;
-    const int64_t threads = (int64_t)ph * M * ((Cout + 3) / 4);
-    hipLaunchKernelGGL(k_conv_fin, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       (const float *)part, pl.ntiles * 16 * NT, pl.ksplit, (const uint16_t *)bias,
-                       (const uint16_t *)res, s_rb, s_rt, (uint16_t *)y, s_yb, s_yt, (int)M, TR, Cout, ph);
-  }
-  return (int)hipGetLastError();
+  const hipError_t e = hipGetLastError();  // (the finish would sum a workspace the main launch never wrote)
+  if (e != hipSuccess || !part) return (int)e;
+  return launch_fin(part, pl.ntiles * 16 * NT, pl.ksplit, bias, res, s_rb, s_rt, y, s_yb, s_yt, M, TR, Cout, ph,
+                    (hipStream_t)stream);
 }
 
 extern "C" int64_t a8_conv_cl_ws_bytes(int B, int TR, int Cin, int Cout, int taps, int ph) {
@@ -724,7 +714,10 @@ extern "C" int64_t a8_conv_cl_ws_bytes(int B, int TR, int Cin, int Cout, int tap
   if (B <= 0 || TR <= 0 || Cin <= 0 || Cout <= 0 || taps <= 0 || ph <= 0) return 0;
   const int64_t M = (int64_t)B * TR;
   if (M > INT32_MAX / 2) return 0;
-  return conv_plan(M, Cin, Cout, taps, ph).ws_bytes;
+  // whichever of the two kernels a call takes (the tile kernel's plan also depends on the call's input rows)
+  const int64_t a = conv_plan(M, Cin, Cout, taps, ph).ws_bytes;
+  const int64_t t = conv_tile_ws_bytes(M, Cin, Cout, taps, ph);
+  return a > t ? a : t;
 }
 
 extern "C" int a8_ru_cl(const void *xin, int64_t s_xb, int64_t s_xt, const void *w1, int64_t s_wt, int64_t s_wc,
@@ -753,6 +746,19 @@ extern "C" int a8_ru_cl(const void *xin, int64_t s_xb, int64_t s_xt, const void 
   if (x_span >= ((int64_t)1 << 31) || w_span >= ((int64_t)1 << 31) || s_xb < 0 || s_xt < 0 || s_wt < 0)
     return set_error(A8_EUNSUP, "ru_cl: xin spans %lld bytes, w1 %lld (each must be below 2 GiB)", (long long)x_span,
                      (long long)w_span);
+  if ((B == 1 || s_xb == (int64_t)Tin * s_xt) && s_xt >= C && s_xt <= 65536 && al16(y) && !((s_yb | s_yt) & 7) &&
+      al16(res) && !((s_rb | s_rt) & 7) && !(reinterpret_cast<uintptr_t>(b2) & 7u)) {
+    const ConvTilePlan tp = conv_tile_plan(M, TR, Tin, C, C, taps, dil, 1, true, false);
+    if (tp.xkb) {
+      ConvTileArgs a{};
+      a.x = (const uint16_t *)xin, a.s_xt = s_xt, a.w = (const uint16_t *)w1, a.s_wt = s_wt, a.s_wc = s_wc;
+      a.bias = (const uint16_t *)b1, a.res = (const uint16_t *)res, a.s_rb = s_rb, a.s_rt = s_rt;
+      a.y = (uint16_t *)y, a.s_yb = s_yb, a.s_yt = s_yt, a.M = (int)M, a.TR = TR, a.Tin = Tin, a.Cin = a.Cout = C;
+      a.taps = taps, a.dil = dil, a.ph = a.ksplit = 1, a.x_span = (uint32_t)x_span, a.w_span = (uint32_t)w_span;
+      a.w2 = (const uint16_t *)w2, a.b2 = (const uint16_t *)b2, a.a2 = a2, a.ib2 = ib2, a.w2_span = (uint32_t)w2_span;
+      return conv_tile_launch(tp, a, true, (hipStream_t)stream);
+    }
+  }
   // the whole row in one tile (NT = C / 16); two row tiles per wave where that still gives >= 512 workgroups
   // (384 channels: one row tile and 32-channel slices, to stay within two workgroups per CU)
   const int WM = C <= 192 && (M + 127) / 128 >= 512 ? 2 : 1;

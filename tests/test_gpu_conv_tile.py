@@ -1,0 +1,82 @@
+"""The tile convolution (csrc/conv_tile.hip) behind conv_cl and ru_cl, where its tiles end: row counts one under, at
+and over its 128 / 192 / 256 / 384 rows, batch rows that divide a tile, do not, or are longer; one to eight taps and
+the widest dilations its LDS slices hold (and one past them, which takes the other kernel); an odd and an even number
+of 96-channel column groups over one or several phases; K split or not; inputs with more rows than the call needs.
+Against the oracle in float64, to one fp16 ulp (fp32 sums in another order) or 1e-3 of the scale where a sum cancels."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+F16 = torch.float16
+
+
+def _close(got, want):
+    g, w = got.cpu().float(), want.float()
+    ulp = (w.abs() * 2 ** -10).clamp(min=2 ** -24)
+    return bool((((g - w).abs() <= ulp * 1.01) | ((g - w).abs() <= 1e-3 * w.abs().max().item())).all())
+
+
+@pytest.mark.parametrize("B,T,extra,Cin,Cout,taps,dil,ph,res,split", [
+    (1, 127, 0, 192, 192, 7, 1, 1, False, True),       # one row under a tile, two column halves
+    (1, 129, 0, 192, 192, 7, 9, 1, True, True),        # one over, the widest dilation
+    (3, 64, 0, 192, 192, 7, 1, 1, True, False),        # batch rows dividing a 192-row tile
+    (7, 50, 0, 192, 384, 7, 3, 1, True, True),         # not dividing it
+    (5, 70, 3, 192, 192, 7, 3, 1, False, True),        # input rows left over after the last tap's reach
+    (37, 4, 0, 512, 192, 7, 1, 1, False, True),        # four-row batch rows: 320-row slices
+    (12, 32, 0, 192, 192, 7, 9, 1, False, True),       # 344-row slices
+    (12, 32, 0, 192, 192, 8, 9, 1, False, True),       # 381-row slices: past the tile kernel's LDS
+    (3, 257, 0, 192, 96, 7, 1, 1, True, True),         # one column group: the 256 / 384-row tile
+    (2, 385, 0, 224, 96, 7, 9, 1, False, True),        #   and 7 channel slices
+    (1, 33, 0, 576, 96, 2, 1, 8, False, True),         # phases in pairs over one column group each
+    (2, 65, 0, 416, 192, 3, 2, 3, True, True),         # six column groups over three phases, 13 channel slices
+    (1, 5, 0, 1152, 96, 1, 1, 3, True, True),          # one tap, an odd number of column groups, one short tile
+    (130, 128, 0, 96, 192, 1, 1, 1, True, False),      # one tap, many tiles (three channel slices)
+    (43, 384, 0, 32, 96, 2, 1, 2, False, False),       # one channel slice, two taps
+])
+def test_conv_tile_edges(a8, dev, B, T, extra, Cin, Cout, taps, dil, ph, res, split):
+    from oracle import conv_ref as cref
+    print(f"case: conv_cl tile B={B} T={T}+{extra} {Cin}->{Cout} taps={taps} dil={dil} ph={ph} res={res} split={split}",
+          flush=True)
+    g = torch.Generator().manual_seed(B + T + Cin + Cout + taps)
+    Tin = T + (taps - 1) * dil + extra
+    x = torch.randn(B, Tin, Cin, generator=g).to(F16)
+    w = (torch.randn(ph, taps, Cin, Cout, generator=g) / (taps * Cin) ** 0.5).to(F16)
+    bv = torch.randn(Cout, generator=g).to(F16)
+    rv = torch.randn(B, T * ph, Cout, generator=g).to(F16) if res else None
+    want = cref.conv_cl(x, w, bv, T, taps, dil, ph, Cout, res=rv)
+    nws = a8.conv_cl_ws_bytes(B, T, Cin, Cout, taps, ph)
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev) if split and nws > 0 else None
+    # rows around the output stay as they are
+    buf = torch.full((B, T * ph + 2, Cout), 7.0, dtype=F16, device=dev)
+    a8.conv_cl(x.to(dev), w.to(dev), bv.to(dev), T, taps, dil, ph, buf[:, 1:T * ph + 1],
+               res=rv.to(dev) if res else None, ws=ws)
+    torch.cuda.synchronize()
+    got = buf.cpu()
+    assert _close(got[:, 1:T * ph + 1], want)
+    assert (got[:, 0] == 7.0).all() and (got[:, T * ph + 1] == 7.0).all()
+
+
+@pytest.mark.parametrize("B,T,C,dil", [(161, 128, 192, 9), (162, 127, 192, 1), (81, 515, 96, 9), (41, 1000, 96, 3)])
+def test_ru_tile_edges(a8, dev, B, T, C, dil):
+    """The residual unit on the tile kernel (enough tiles for it): full and ragged tiles, both widths."""
+    from oracle import conv_ref as cref
+    print(f"case: ru_cl tile B={B} T={T} C={C} dil={dil}", flush=True)
+    g = torch.Generator().manual_seed(B * 7 + C + dil)
+    taps, ctx = 7, 6 * dil
+    x = torch.randn(B, T, C, generator=g).half()
+    st = torch.randn(B, ctx, C, generator=g).half()
+    a1, a2 = torch.rand(C, generator=g) + 0.5, torch.rand(C, generator=g) + 0.5
+    ib1, ib2 = 1.0 / (a1 + 1e-9), 1.0 / (a2 + 1e-9)
+    w1 = (torch.randn(taps, C, C, generator=g) / (taps * C) ** 0.5).half()
+    w2 = (torch.randn(C, C, generator=g) / C ** 0.5).half()
+    b1, b2 = (0.1 * torch.randn(C, generator=g)).half(), (0.1 * torch.randn(C, generator=g)).half()
+    want = cref.ru_fused(x, st, a1, ib1, w1, b1, a2, ib2, w2, b2, taps, dil)
+    xd = x.to(dev)
+    xin = torch.empty(B, ctx + T, C, dtype=F16, device=dev)
+    a8.snake_cat(xd, st.to(dev), a1.to(dev), ib1.to(dev), xin)
+    out = torch.full((B, T, C), 9.0, dtype=F16, device=dev)
+    a8.ru_cl(xin, w1.to(dev), b1.to(dev), a2.to(dev), ib2.to(dev), w2.to(dev), b2.to(dev), xd, out, T, taps, dil)
+    torch.cuda.synchronize()
+    assert _close(out, want)
