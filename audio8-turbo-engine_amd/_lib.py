@@ -71,6 +71,12 @@ SIGNATURES = {
                                  _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P]),
 }
 
+# the vocoder's own entry points; mirrors include/a8voc.h
+VOC_SIGNATURES = {
+    "a8_conv_cl_snake": (_I, [_P, _L, _L, _P, _L, _L, _L, _I, _P, _P, _L, _L, _P, _L, _L, _P, _P, _P, _P,
+                              _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P]),
+}
+
 _lock = threading.Lock()
 _lib = None
 
@@ -90,7 +96,7 @@ def load() -> ctypes.CDLL:
                 raise ImportError(f"{LIB_PATH} is missing: build it with `python __graft_entry__.py build` "
                                   "(or __graft_entry__.build()) before using the HIP kernels")
             lib = ctypes.CDLL(LIB_PATH)
-            for name, (res, args) in SIGNATURES.items():
+            for name, (res, args) in (*SIGNATURES.items(), *VOC_SIGNATURES.items()):
                 fn = getattr(lib, name)
                 fn.restype, fn.argtypes = res, args
             _lib = lib

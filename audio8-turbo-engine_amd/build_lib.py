@@ -41,12 +41,12 @@ SOURCE_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 
 
 def source_hash() -> str:
-    """A short hash of every source the library is built from (csrc/ and include/a8attn.h); the build bakes it
+    """A short hash of every source the library is built from (csrc/ and include/); the build bakes it
     into a8_version(), so a library older than its sources can be told apart."""
     import hashlib
     h = hashlib.sha1()
-    inc = os.path.join(os.path.dirname(HERE), "include", "a8attn.h")
-    for p in sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC)) + [inc]:
+    inc = os.path.join(os.path.dirname(HERE), "include")
+    for p in sorted(os.path.join(d, f) for d in (CSRC, inc) for f in os.listdir(d)):
         if os.path.isfile(p):
             h.update(os.path.basename(p).encode())
             with open(p, "rb") as f:

@@ -30,6 +30,7 @@
 //     order by a finishing kernel, so results do not depend on timing.
 // The snake's sine runs on the hardware sine unit after an exact reduction to one period.
 // snake_cat: one lane per 8 channels of one output row, 16-byte loads and stores.
+#include "../../include/a8voc.h"
 #include "conv_tile.h"
 #include "fp16_ops.h"
 
@@ -52,6 +53,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_cl(const uint16_t *__restrict__
                                                  uint32_t w_span, const uint16_t *__restrict__ w2,
                                                  const uint16_t *__restrict__ b2, const float *__restrict__ a2,
                                                  const float *__restrict__ ib2, uint32_t w2_span) {
+  // a2 / ib2 without RU: a snake over the stored (fp16) outputs, or null
   warm_kernargs<220>();  // the explicit arguments above span 0x00-0xdb
   static_assert(!RU || (!SNAKE && NT % 2 == 0), "residual unit: input pre-activated, 32-channel k steps");
   constexpr int BN = 16 * NT, BM = 64 * WM, KS = 32 * KSUB, NCH = BN / 8;
@@ -297,14 +299,18 @@ __global__ __launch_bounds__(256, 2) void k_conv_cl(const uint16_t *__restrict__
           const u32x2 rv = ld8(rrow + n);
           v[0] += h_lo(rv[0]), v[1] += h_hi(rv[0]), v[2] += h_lo(rv[1]), v[3] += h_hi(rv[1]);
         }
-        st8(yrow + n, u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])});
+        u32x2 o = u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+        if (!RU && a2) o = snake4(o, a2 + n, ib2 + n);
+        st8(yrow + n, o);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (n + e >= Cout) continue;
           if (bias) v[e] += h_lo(bias[n + e]);
           if (rrow) v[e] += h_lo(rrow[n + e]);
-          yrow[n + e] = (uint16_t)(pack_f16x2(v[e], 0.f) & 0xffffu);
+          uint32_t o = pack_f16x2(v[e], 0.f);
+          if (!RU && a2) o = snake2(o, a2[n + e], ib2[n + e], 0.f, 0.f);
+          yrow[n + e] = (uint16_t)(o & 0xffffu);
         }
       }
     }
@@ -316,8 +322,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_cl(const uint16_t *__restrict__
 __global__ __launch_bounds__(256) void k_conv_fin(const float *__restrict__ part, int64_t NP, int ksplit,
                                                   const uint16_t *__restrict__ bias, const uint16_t *__restrict__ res,
                                                   int64_t s_rb, int64_t s_rt, uint16_t *__restrict__ y, int64_t s_yb,
-                                                  int64_t s_yt, int M, int TR, int Cout, int PH) {
-  warm_kernargs<92>();  // the explicit arguments above span 0x00-0x5b
+                                                  int64_t s_yt, int M, int TR, int Cout, int PH,
+                                                  const float *__restrict__ oa, const float *__restrict__ oib) {
+  warm_kernargs<112>();  // the explicit arguments above span 0x00-0x6f
   const int nq = (Cout + 3) >> 2;
   const uint32_t id = blockIdx.x * 256u + threadIdx.x;
   if (id >= (uint32_t)PH * (uint32_t)M * (uint32_t)nq) return;
@@ -334,7 +341,9 @@ __global__ __launch_bounds__(256) void k_conv_fin(const float *__restrict__ part
     float o = v[e];
     if (bias) o += h_lo(bias[n + e]);
     if (res) o += h_lo(res[(int64_t)b * s_rb + orow * s_rt + n + e]);
-    y[(int64_t)b * s_yb + orow * s_yt + n + e] = (uint16_t)(pack_f16x2(o, 0.f) & 0xffffu);
+    uint32_t ov = pack_f16x2(o, 0.f);
+    if (oa) ov = snake2(ov, oa[n + e], oib[n + e], 0.f, 0.f);
+    y[(int64_t)b * s_yb + orow * s_yt + n + e] = (uint16_t)(ov & 0xffffu);
   }
 }
 
@@ -573,21 +582,22 @@ static ConvPlan conv_plan(int64_t M, int Cin, int Cout, int taps, int ph, bool a
 // k_conv_fin over the partials of `ksplit` shares, rows of NP floats.
 static int launch_fin(const float *part, int64_t NP, int ksplit, const void *bias, const void *res, int64_t s_rb,
                       int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, int64_t M, int TR, int Cout, int ph,
-                      hipStream_t stream) {
+                      const float *oa, const float *oib, hipStream_t stream) {
   const int64_t threads = (int64_t)ph * M * ((Cout + 3) / 4);
   hipLaunchKernelGGL(k_conv_fin, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, part, NP, ksplit,
                      (const uint16_t *)bias, (const uint16_t *)res, s_rb, s_rt, (uint16_t *)y, s_yb, s_yt, (int)M, TR,
-                     Cout, ph);
+                     Cout, ph, oa, oib);
   return (int)hipGetLastError();
 }
 
 }  // namespace a8
 
-extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void *w, int64_t s_wp, int64_t s_wt,
-                          int64_t s_wc, int cout_w, const void *bias, const void *res, int64_t s_rb, int64_t s_rt,
-                          void *y, int64_t s_yb, int64_t s_yt, const float *snake_a, const float *snake_ib, int B,
-                          int Tin, int TR, int Cin, int Cout, int taps, int dil, int ph, void *ws, int64_t ws_bytes,
-                          void *stream) {
+extern "C" int a8_conv_cl_snake(const void *x, int64_t s_xb, int64_t s_xt, const void *w, int64_t s_wp, int64_t s_wt,
+                                int64_t s_wc, int cout_w, const void *bias, const void *res, int64_t s_rb,
+                                int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, const float *snake_a,
+                                const float *snake_ib, const float *out_a, const float *out_ib, int B, int Tin, int TR,
+                                int Cin, int Cout, int taps, int dil, int ph, void *ws, int64_t ws_bytes,
+                                void *stream) {
   using namespace a8;
   if (B < 0 || TR < 0 || Cin <= 0 || Cout <= 0 || taps <= 0 || dil <= 0 || ph <= 0 || cout_w < Cout)
     return set_error(A8_EINVAL, "conv_cl: bad sizes B=%d TR=%d Cin=%d Cout=%d taps=%d dil=%d ph=%d cout_w=%d", B, TR,
@@ -598,13 +608,13 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
   if (snake_a && Cin > kSnakeMaxC)
     return set_error(A8_EUNSUP, "conv_cl: the snake on the load takes Cin <= %d (got %d; use snake_cat)", kSnakeMaxC, Cin);
   if (B == 0 || TR == 0) return 0;
-  if (!x || !w || !y || (snake_a != nullptr) != (snake_ib != nullptr))
+  if (!x || !w || !y || (snake_a != nullptr) != (snake_ib != nullptr) || (out_a != nullptr) != (out_ib != nullptr))
     return set_error(A8_EINVAL, "conv_cl: null pointer");
   // y (and res) may be any 2-byte-aligned view: the epilogue stores element by element unless 8-byte stores of
   // four channels are aligned. The weight rows are read 16 bytes at a time: cout_w (its padded width) must be a
   // multiple of 8.
   if (!al16(x) || !al16(w) || (s_xb | s_xt | s_wp | s_wt | s_wc) & 7 || (cout_w & 7) ||
-      (snake_a && (!al16(snake_a) || !al16(snake_ib))) || (reinterpret_cast<uintptr_t>(y) & 1u) ||
+      (snake_a && (!al16(snake_a) || !al16(snake_ib))) || (out_a && (!al16(out_a) || !al16(out_ib))) || (reinterpret_cast<uintptr_t>(y) & 1u) ||
       (res && (reinterpret_cast<uintptr_t>(res) & 1u)))
     return set_error(A8_EALIGN, "conv_cl: x / w / snake 16-byte aligned, their strides and the weight's padded "
                      "width (%d) multiples of 8", cout_w);
@@ -633,11 +643,11 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
       a.bias = (const uint16_t *)bias, a.res = (const uint16_t *)res, a.s_rb = s_rb, a.s_rt = s_rt;
       a.y = (uint16_t *)y, a.s_yb = s_yb, a.s_yt = s_yt, a.M = (int)M, a.TR = TR, a.Tin = Tin, a.Cin = Cin;
       a.Cout = Cout, a.taps = taps, a.dil = dil, a.ph = ph, a.part = tp.ksplit > 1 ? (float *)ws : nullptr;
-      a.ksplit = tp.ksplit, a.x_span = (uint32_t)x_span, a.w_span = (uint32_t)w_span;
+      a.oa = out_a, a.oib = out_ib, a.ksplit = tp.ksplit, a.x_span = (uint32_t)x_span, a.w_span = (uint32_t)w_span;
       const int e = conv_tile_launch(tp, a, false, (hipStream_t)stream);
       if (e || tp.ksplit == 1) return e;
       return launch_fin((const float *)ws, Cout, tp.ksplit, bias, res, s_rb, s_rt, y, s_yb, s_yt, M, TR, Cout, ph,
-                        (hipStream_t)stream);
+                        out_a, out_ib, (hipStream_t)stream);
     }
   }
   const int NT = pl.NT, WM = pl.WM;
@@ -646,7 +656,7 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
 #define A8_CONV_ARGS (const uint16_t *)x, s_xb, s_xt, (const uint16_t *)w, s_wp, s_wt, s_wc, (const uint16_t *)bias, \
                      (const uint16_t *)res, s_rb, s_rt, (uint16_t *)y, s_yb, s_yt, snake_a, snake_ib, (int)M, TR, Cin, \
                      Cout, cout_w, taps, dil, ph, part, pl.ksplit, (uint32_t)x_span, (uint32_t)w_span, nullptr,     \
-                     nullptr, nullptr, nullptr, 0u
+                     nullptr, out_a, out_ib, 0u
 #define A8_CONV_L(wm, nt, ksub, sn) \
   hipLaunchKernelGGL((k_conv_cl<wm, nt, ksub, sn>), grid, dim3(256), 0, (hipStream_t)stream, A8_CONV_ARGS)
 #define A8_CONV_NT(wm, ksub, sn)                 \
@@ -706,7 +716,16 @@ extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void 
   const hipError_t e = hipGetLastError();  // (the finish would sum a workspace the main launch never wrote)
   if (e != hipSuccess || !part) return (int)e;
   return launch_fin(part, pl.ntiles * 16 * NT, pl.ksplit, bias, res, s_rb, s_rt, y, s_yb, s_yt, M, TR, Cout, ph,
-                    (hipStream_t)stream);
+                    out_a, out_ib, (hipStream_t)stream);
+}
+
+extern "C" int a8_conv_cl(const void *x, int64_t s_xb, int64_t s_xt, const void *w, int64_t s_wp, int64_t s_wt,
+                          int64_t s_wc, int cout_w, const void *bias, const void *res, int64_t s_rb, int64_t s_rt,
+                          void *y, int64_t s_yb, int64_t s_yt, const float *snake_a, const float *snake_ib, int B,
+                          int Tin, int TR, int Cin, int Cout, int taps, int dil, int ph, void *ws, int64_t ws_bytes,
+                          void *stream) {
+  return a8_conv_cl_snake(x, s_xb, s_xt, w, s_wp, s_wt, s_wc, cout_w, bias, res, s_rb, s_rt, y, s_yb, s_yt, snake_a,
+                          snake_ib, nullptr, nullptr, B, Tin, TR, Cin, Cout, taps, dil, ph, ws, ws_bytes, stream);
 }
 
 extern "C" int64_t a8_conv_cl_ws_bytes(int B, int TR, int Cin, int Cout, int taps, int ph) {

@@ -24,6 +24,7 @@ struct ConvTileArgs {
   const uint16_t *w2, *b2;
   const float *a2, *ib2;
   uint32_t w2_span;
+  const float *oa, *oib;  // a snake over the stored (fp16) outputs, or null
 };
 
 // mt: 32-row groups of a wave. xkb: KiB of LDS one 32-channel slice of a tile's input rows takes (16 rows a KiB); 0:

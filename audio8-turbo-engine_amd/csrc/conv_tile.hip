@@ -319,7 +319,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_tile(const ConvTileArgs a) {
         uint32_t o2 = pack_f16x2(v[4], v[5]), o3 = pack_f16x2(v[6], v[7]);
         swap32(o0, o2);
         swap32(o1, o3);
-        if (ok) st16(yrow + 32 * nt + 16 * qq, u32x4{o0, o1, o2, o3});
+        u32x4 o = u32x4{o0, o1, o2, o3};
+        if (a.oa) o = snake8(o, a.oa + nb + 32 * nt + 16 * qq + 8 * h, a.oib + nb + 32 * nt + 16 * qq + 8 * h);
+        if (ok) st16(yrow + 32 * nt + 16 * qq, o);
       }
   }
 }

@@ -81,19 +81,21 @@ class CLConv:
             if need > 0:
                 self.ws = torch.empty(need, dtype=torch.uint8, device=dev)
 
-    def __call__(self, x, b, res=None):
-        """x [b, T, Cin] fp16 (pre-activation) -> [b, T*ph, Cout] fp16."""
+    def __call__(self, x, b, res=None, out_snake=None, activated=False):
+        """x [b, T, Cin] fp16 (pre-activation) -> [b, T*ph, Cout] fp16. out_snake: the next conv's (alpha, ib), applied
+        to the outputs as they are stored; activated (a conv without state): x has this conv's snake applied already."""
         T = x.shape[1]
         y = torch.empty(b, T * self.ph, self.Cout, dtype=F16, device=x.device)
         if self.state is None:
-            snake = (self.a, self.ib) if self.a is not None else None
+            snake = (self.a, self.ib) if self.a is not None and not activated else None
             conv_cl(x.contiguous(), self.W, self.bias, T, self.taps, self.dil, self.ph, y, res=res, snake=snake,
-                    ws=self.ws)
+                    ws=self.ws, out_snake=out_snake)
             return y
         xin = torch.empty(b, self.ctx + T, self.Cin, dtype=F16, device=x.device)
         refresh = T >= self.ctx  # the next context written by snake_cat itself (no copy after the conv)
         snake_cat(x, self.state[:b], self.a, self.ib, xin, refresh=refresh)
-        conv_cl(xin, self.W, self.bias, T, self.taps, self.dil, self.ph, y, res=res, ws=self.ws)
+        conv_cl(xin, self.W, self.bias, T, self.taps, self.dil, self.ph, y, res=res, ws=self.ws,
+                out_snake=out_snake)
         if not refresh:
             self.state[:b].copy_(xin[:, T:])
         return y
@@ -209,7 +211,15 @@ class CLDecoder:
         for tc, units in self.blocks:
             x = tc(x, b)
             for c1, c2, fu in units:
-                x = fu(x, b) if fu is not None else c2(c1(x, b), b, res=x)
+                if fu is not None:
+                    x = fu(x, b)
+                elif c2.state is None and c2.a is not None:
+                    # c1's output feeds c2 alone, so c2's snake is applied as c1 stores it: once an element (c2's
+                    # column tiles each applied it on their loads), and c2 runs on the tile kernel, which has no
+                    # snake on its loads
+                    x = c2(c1(x, b, out_snake=(c2.a, c2.ib)), b, res=x, activated=True)
+                else:
+                    x = c2(c1(x, b), b, res=x)
         f = self.final
         if self.fused_out and x.shape[1] >= f.ctx:
             y = torch.empty(b, x.shape[1], dtype=torch.float32, device=x.device)

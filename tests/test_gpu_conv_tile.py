@@ -80,3 +80,35 @@ def test_ru_tile_edges(a8, dev, B, T, C, dil):
     a8.ru_cl(xin, w1.to(dev), b1.to(dev), a2.to(dev), ib2.to(dev), w2.to(dev), b2.to(dev), xd, out, T, taps, dil)
     torch.cuda.synchronize()
     assert _close(out, want)
+
+
+@pytest.mark.parametrize("B,T,Cin,Cout,cw,taps,split", [
+    (3, 64, 192, 192, 192, 7, False),   # the tile kernel
+    (3, 64, 192, 192, 192, 7, True),    #   K split: in the finish
+    (3, 40, 64, 96, 96, 3, False),      # k_conv_cl: four channels a store
+    (3, 40, 64, 30, 32, 3, False),      #   element by element
+    (4, 8, 512, 30, 32, 7, True),       #   K split
+])
+def test_out_snake_equals_a_snake_pass(a8, dev, B, T, Cin, Cout, cw, taps, split):
+    """conv_cl with out_snake against conv_cl then the snake over its fp16 outputs (snake_cat without a context; per
+    channel, so Cout is padded to whole 16-byte chunks there): the same bits."""
+    print(f"case: out_snake B={B} T={T} {Cin}->{Cout} taps={taps} split={split}", flush=True)
+    g = torch.Generator().manual_seed(Cin + Cout + taps)
+    x = (torch.randn(B, T + taps - 1, Cin, generator=g)).to(F16).to(dev)
+    w = (torch.randn(1, taps, Cin, cw, generator=g) / (taps * Cin) ** 0.5).to(F16).to(dev)
+    bv = torch.randn(cw, generator=g).to(F16).to(dev)
+    oa = torch.rand(cw, generator=g).to(dev) + 0.5
+    oib = 1.0 / (oa + 1e-9)
+    nws = a8.conv_cl_ws_bytes(B, T, Cin, Cout, taps, 1)
+    assert not split or nws > 0
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev) if split else None
+    y = torch.empty(B, T, Cout, dtype=F16, device=dev)
+    plain = torch.zeros(B, T, cw, dtype=F16, device=dev)
+    a8.conv_cl(x, w, bv, T, taps, 1, 1, y, ws=ws, out_snake=(oa, oib))
+    tight = torch.empty(B, T, Cout, dtype=F16, device=dev)
+    a8.conv_cl(x, w, bv, T, taps, 1, 1, tight, ws=ws)
+    plain[..., :Cout] = tight
+    want = torch.empty_like(plain)
+    a8.snake_cat(plain, None, oa, oib, want)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want[..., :Cout])
