@@ -117,9 +117,17 @@ def check(status: int, what: str) -> None:
     raise A8Error(f"{what}: HIP error {status}")
 
 
+def _raw_stream_of_device(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# torch's own accessor of the current stream's handle, without a Stream object per call
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or _raw_stream_of_device
+
+
 def stream_of(t: torch.Tensor) -> int:
     """hipStream_t (as an int) of torch's current stream on t's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def version() -> str:

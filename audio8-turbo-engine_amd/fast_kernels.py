@@ -32,7 +32,13 @@ def _need(cond: bool, msg: str, exc=ValueError):
         raise exc(msg)
 
 
+# The checks of every call: one condition on what passes, and the messages (formatting them costs more than the
+# checks) only for what does not. With them prefix_copy's host time per call is below its 12 us on the GPU: an
+# admission of 64 slots (4 calls, eager) 73 -> 48 us.
 def _check_bf16(name: str, t: torch.Tensor, dims: int):
+    if (isinstance(t, torch.Tensor) and t.dtype == _BF16 and t.dim() == dims and
+            (t.stride(-1) == 1 or t.shape[-1] == 1)):
+        return
     _need(isinstance(t, torch.Tensor), f"{name} must be a tensor", TypeError)
     _need(t.dtype == _BF16, f"{name} must be bfloat16 (got {t.dtype})", TypeError)
     _need(t.dim() == dims, f"{name} must have {dims} dims (got shape {tuple(t.shape)})")
@@ -40,6 +46,9 @@ def _check_bf16(name: str, t: torch.Tensor, dims: int):
 
 
 def _check_i32(name: str, t: torch.Tensor, n: int):
+    if (isinstance(t, torch.Tensor) and t.dtype == _I32 and t.dim() == 1 and t.is_contiguous() and
+            t.shape[0] >= n):
+        return
     _need(isinstance(t, torch.Tensor), f"{name} must be a tensor", TypeError)
     _need(t.dtype == _I32, f"{name} must be int32 (got {t.dtype})", TypeError)
     _need(t.dim() == 1 and t.is_contiguous(), f"{name} must be a contiguous 1-D tensor")
@@ -48,6 +57,16 @@ def _check_i32(name: str, t: torch.Tensor, n: int):
 
 def _check_device(**tensors):
     """Every tensor on one HIP device (the kernels dereference all of them there)."""
+    first = -1
+    for t in tensors.values():
+        if t is not None:
+            d = t.get_device() if t.is_cuda else -1
+            if d < 0 or (first >= 0 and d != first):
+                break
+            first = d
+    else:
+        if first >= 0:
+            return
     devs = {t.device for t in tensors.values() if t is not None}
     for name, t in tensors.items():
         _need(t is None or t.is_cuda, f"{name} must be on a HIP device (got {t.device if t is not None else None})")
@@ -506,9 +525,11 @@ def prefix_copy(k, v, kc_all, vc_all, slots):
     _need(kc_all.shape == vc_all.shape and kc_all.stride() == vc_all.stride(),
           "kc_all and vc_all must have the same shape and strides")
     layers, nkv, Lp, hd = k.shape
-    _need(kc_all.shape[0] == layers and kc_all.shape[2] == nkv and kc_all.shape[4] == hd,
-          f"cache shape {tuple(kc_all.shape)} does not match [{layers}, rows, {nkv}, S, {hd}]")
-    _need(Lp <= kc_all.shape[3], f"prefix of {Lp} positions does not fit a cache of {kc_all.shape[3]}")
+    c_layers, c_rows, c_nkv, S, c_hd = kc_all.shape
+    if c_layers != layers or c_nkv != nkv or c_hd != hd:
+        raise ValueError(f"cache shape {tuple(kc_all.shape)} does not match [{layers}, rows, {nkv}, S, {hd}]")
+    if Lp > S:
+        raise ValueError(f"prefix of {Lp} positions does not fit a cache of {S}")
     if not isinstance(slots, torch.Tensor):
         slots = torch.tensor(list(slots), dtype=_I32)
         if kc_all.is_cuda:
@@ -518,10 +539,11 @@ def prefix_copy(k, v, kc_all, vc_all, slots):
     n = slots.shape[0]
     if n == 0 or layers == 0 or Lp == 0:
         return
+    s_l, s_h, s_p, _ = k.stride()
+    d_l, d_r, d_h, d_p, _ = kc_all.stride()
     st = _lib.load().a8_prefix_copy(
-        k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
-        kc_all.data_ptr(), vc_all.data_ptr(), kc_all.stride(0), kc_all.stride(1), kc_all.stride(2), kc_all.stride(3),
-        slots.data_ptr(), n, layers, nkv, Lp, hd, kc_all.shape[1], kc_all.shape[3], _lib.stream_of(kc_all))
+        k.data_ptr(), v.data_ptr(), s_l, s_h, s_p, kc_all.data_ptr(), vc_all.data_ptr(), d_l, d_r, d_h, d_p,
+        slots.data_ptr(), n, layers, nkv, Lp, hd, c_rows, S, _lib.stream_of(kc_all))
     _lib.check(st, "prefix_copy")
 
 
