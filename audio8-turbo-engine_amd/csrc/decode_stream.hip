@@ -23,6 +23,7 @@
 //     need a device-scope handshake per chunk (store completion, counter atomic, partial reads): on a
 //     saturated memory system each of those round trips waits microseconds in the same queues the
 //     KV stream fills, which costs far more than the extra launch.
+#include "decode_short.h"
 #include "decode_tile.h"
 #include "rope.h"
 
@@ -477,6 +478,13 @@ static int stream_entry(const char *fn, const void *q, int64_t s_qb, int64_t s_q
                     rows_launch(grid, st, qq, s_qb, s_qh, kk, vv, s_kb, s_kh, cache_rows, cache_len, lens, rowmap, oo,
                                 s_ob, s_oh, b, nq, nkv, group, sl2, si);
   if (rows) return (int)hipGetLastError();
+  // a fused launch over a cache of at most half a tile: k_decode_short (the same bits); phases bit 2 keeps
+  // k_decode_stream here too
+  if (fused && (phases & 1) && !(phases & 4) && P == 1 && cache_len <= kShortKeys) {
+    hipLaunchKernelGGL(k_decode_short, dim3((unsigned)(b * nkv)), dim3(64), 0, st, kk, vv, s_kb, s_kh, cache_rows,
+                       cache_len, lens, rowmap, oo, s_ob, s_oh, b, nq, nkv, group, sl2, si);
+    return (int)hipGetLastError();
+  }
   if (phases & 1) {
 #define A8_STREAM_ARGS grid, st, qq, s_qb, s_qh, kk, vv, s_kb, s_kh, s_ks, cache_rows, cache_len, lens, rowmap, oo, \
                        s_ob, s_oh, acc_ws, ml_ws, b, nq, nkv, group, tiles_per_wave, P, sl2, si
