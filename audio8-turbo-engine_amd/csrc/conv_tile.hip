@@ -23,8 +23,8 @@
 // Against k_conv_cl (each wave the whole column width of 16 or 32 rows, X operands from memory again for every tap;
 // graph replays, 192 batch rows of 4 frames): 384 channels k 7 131 -> 94 us (1.08 PFLOP/s; a large fp16 matrix product
 // on this card: 1.45), 768 channels k 7 92 -> 72, the stride-8 transposed convs 78 -> 46 and 83 -> 61, stride 4
-// 96 -> 70, stride 2 77 -> 48, the input conv 51 -> 37; the residual units of 192 / 96 channels 171 -> 139 and
-// 112 -> 90 (64-row waves). 24 batch rows: 37 -> 32, 25 -> 24, 20 -> 20, 34 -> 25, 28 -> 17, 14 -> 12.6, 25.5 -> 20.
+// 96 -> 70, stride 2 77 -> 48, the input conv 51 -> 37; the residual units of 192 / 96 channels 172 -> 135 and
+// 114 -> 88 (64-row waves, the two column halves' whole rows exchanged at once: 141 and 92). 24 batch rows: 37 -> 32, 25 -> 24, 20 -> 20, 34 -> 25, 28 -> 17, 14 -> 12.6, 25.5 -> 20.
 #include "conv_tile.h"
 
 #include "fp16_ops.h"
@@ -33,7 +33,6 @@ namespace a8 {
 
 namespace {
 
-constexpr int kRuMt = 2;              // row groups a wave of a residual unit's tile
 constexpr int kHalf = 32 * 96 * 2;  // bytes of a W slice's column half
 
 typedef uint32_t rsrc_words_t __attribute__((ext_vector_type(4)));
@@ -74,7 +73,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_tile(const ConvTileArgs a) {
   constexpr int NH = 4 / WMW, BM = 32 * MT * WMW;
   constexpr int kW = NH * kHalf, kWI = NH * 6;          // a W slice: bytes, DMA instructions
   constexpr int WR = (kWI + 3) / 4, XI = (XKB + 3) / 4;  // instructions per wave and slice (the last repeated)
-  constexpr int kMainLds = 3 * kW + 2 * XKB * 1024, kRuLds = (NH == 2 ? 2 * MT * 12 * 1024 : 0) + 2 * kW;
+  constexpr int kMainLds = 3 * kW + 2 * XKB * 1024, kRuLds = (NH == 2 ? 2 * 8 * MT * 1024 : 0) + 2 * kW;
   constexpr int kLds = RU && kRuLds > kMainLds ? kRuLds : kMainLds;
   static_assert(kLds <= 80 * 1024, "two workgroups per compute unit");
   __shared__ __attribute__((aligned(16))) char smem[kLds];
@@ -228,35 +227,49 @@ __global__ __launch_bounds__(256, 2) void k_conv_tile(const ConvTileArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[nt][i][e] = 0.f;
     const rsrc_words_t w2r = rsrc_words(a.w2, a.w2_span);
-    auto w2_off = [&](int kc) __attribute__((always_inline)) -> uint32_t { return (uint32_t)((int64_t)kc * 32 * a.s_wc * 2); };
     const int aoff2 = wn * kHalf + (4 * h + (l15 >> 2)) * 192 + (16 * ((lane >> 4) & 1) + 4 * (l15 & 3)) * 2;
-    constexpr int S2 = 3 * NH;                          // 32-channel slices of w2
-    constexpr int kH = NH == 2 ? 2 * MT * 12 * 1024 : 0;  // the exchange area: h of the tile's 32-row groups
-    lds_barrier();  // every wave is done with the ring
-    issue_w(w2r, kH, w2_off(0));
-    if constexpr (NH == 2) {  // a row's channels lie in two waves: through LDS, in operand order
+    constexpr int S2 = 3 * NH;  // 32-channel steps over the row
+    // Two column halves: a wave holds half of its rows' channels, its partner (wave ^ 1) the other half. It starts
+    // with its own three slices, from registers, then takes the partner's through LDS, a 32-channel slice at a time
+    // (two slice areas: the third goes out once the first has been read everywhere). So in step s2 column half hh
+    // multiplies w2's rows of slice 3 hh + s2, then of slice 3 (1 - hh) + s2 - 3.
+    constexpr int kEx = 8 * MT * 1024, kH = NH == 2 ? 2 * kEx : 0;
+    auto issue_w2 = [&](int s2, int slot) __attribute__((always_inline)) {
 #pragma unroll
-      for (int s = 0; s < 6; ++s)
+      for (int i = 0; i < WR; ++i) {
+        const int half = wq[i] / 6;
+        const int slice = NH == 1 ? s2 : s2 < 3 ? 3 * half + s2 : 3 * (1 - half) + s2 - 3;
+        dma16(w2r, lds0 + kH + slot * kW + wq[i] * 1024, wvo[i], (uint32_t)((int64_t)slice * 32 * a.s_wc * 2));
+      }
+    };
+    auto ex_at = [&](int c, int wave, int u, int i) __attribute__((always_inline)) {
+      return smem + (c & 1) * kEx + (((wave * 2 + u) * MT + i) * 64 + lane) * 16;
+    };
+    auto ex_put = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          *(__attribute__((address_space(3))) u32x4 *)(smem + (((MT * wm + i) * 12 + 6 * wn + s) * 64 + lane) * 16) = hb[s][i];
+          *(__attribute__((address_space(3))) u32x4 *)ex_at(c, wv, u, i) = hb[2 * c + u][i];
+    };
+    lds_barrier();  // every wave is done with the ring
+    issue_w2(0, 0);
+    if constexpr (NH == 2) {
+      ex_put(0);
+      ex_put(1);
     }
 #pragma unroll
     for (int s2 = 0; s2 < S2; ++s2) {
       wait_vmcnt<0>();
       lds_barrier();
-      if (s2 + 1 < S2) issue_w(w2r, kH + ((s2 + 1) & 1) * kW, w2_off(s2 + 1));
+      if (s2 + 1 < S2) issue_w2(s2 + 1, (s2 + 1) & 1);
+      if (NH == 2 && s2 == 4) ex_put(2);
       const char *wp = smem + kH + (s2 & 1) * kW + aoff2;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         u32x4 bx[MT];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-          if constexpr (NH == 2)
-            bx[i] = lds_ld16(smem + (((MT * wm + i) * 12 + 2 * s2 + u) * 64 + lane) * 16);
-          else
-            bx[i] = hb[2 * s2 + u][i];
-        }
+        for (int i = 0; i < MT; ++i) bx[i] = s2 < 3 ? hb[(2 * s2 + u) % 6][i] : lds_ld16(ex_at(s2 - 3, wv ^ 1, u, i));
 #pragma unroll
         for (int nt = 0; nt < 3; ++nt) {
           const u32x2 lo = lds_tr16(wp + u * 16 * 192 + nt * 64), hi = lds_tr16(wp + u * 16 * 192 + nt * 64 + 8 * 192);
@@ -384,7 +397,6 @@ ConvTilePlan conv_tile_plan(int64_t M, int TR, int Tin, int Cin, int Cout, int t
   pl.narrow = ph * (Cout / 96) % 2 != 0;
   double best = 0;
   for (int mt = 2; mt <= 3; ++mt) {
-    if (ru && mt != kRuMt) continue;
     const int xkb = tile_xkb(TR, Tin, taps, dil, pl.narrow, ru, mt);
     if (!xkb) continue;
     double us;
@@ -413,10 +425,10 @@ static int launch(const ConvTileArgs &a, hipStream_t stream) {
 
 int conv_tile_launch(const ConvTilePlan &pl, const ConvTileArgs &a, bool ru, hipStream_t stream) {
   if (pl.narrow) {
-    if (ru) return launch<4, 2, 20, true>(a, stream);
+    if (ru) return pl.mt == 3 ? launch<4, 3, 28, true>(a, stream) : launch<4, 2, 20, true>(a, stream);
     return pl.mt == 3 ? launch<4, 3, 28, false>(a, stream) : launch<4, 2, 20, false>(a, stream);
   }
-  if (ru) return launch<2, 2, 12, true>(a, stream);
+  if (ru) return pl.mt == 3 ? launch<2, 3, 16, true>(a, stream) : launch<2, 2, 12, true>(a, stream);
   if (pl.mt == 3) return pl.xkb == 16 ? launch<2, 3, 16, false>(a, stream) : launch<2, 3, 22, false>(a, stream);
   return pl.xkb == 12 ? launch<2, 2, 12, false>(a, stream) : launch<2, 2, 22, false>(a, stream);
 }
