@@ -318,7 +318,10 @@ __global__ __launch_bounds__(256, 2) void k_conv_cl(const uint16_t *__restrict__
 }
 
 // Split-K finish: Y = sum over ks of part[ks] (in ks order) + bias (+ res), one rounding to fp16; one thread per
-// 4 channels of one output row.
+// 4 channels of one output row. Bounded by its start and one round trip where the partials are few (they come eight
+// shares at a time, in flight together: added one by one as they were loaded, each share was a round trip), by memory
+// where they are many; VEC (channels in fours, 8-byte aligned rows): 8-byte residual loads and stores.
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_conv_fin(const float *__restrict__ part, int64_t NP, int ksplit,
                                                   const uint16_t *__restrict__ bias, const uint16_t *__restrict__ res,
                                                   int64_t s_rb, int64_t s_rt, uint16_t *__restrict__ y, int64_t s_yb,
@@ -331,19 +334,44 @@ __global__ __launch_bounds__(256) void k_conv_fin(const float *__restrict__ part
   const int c = (int)(id % (uint32_t)nq);
   const uint32_t pm = id / (uint32_t)nq;
   const int m = (int)(pm % (uint32_t)M), p = (int)(pm / (uint32_t)M), n = 4 * c;
-  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < ksplit; ++k) v += *reinterpret_cast<const f32x4 *>(part + ((int64_t)(k * PH + p) * M + m) * NP + n);
   const int b = m / TR, t = m - b * TR;
   const int64_t orow = (int64_t)t * PH + p;
+  const uint16_t *rp = res ? res + (int64_t)b * s_rb + orow * s_rt + n : nullptr;
+  u32x2 rv = u32x2{0u, 0u}, bv = u32x2{0u, 0u};
+  if (VEC) {
+    if (rp) rv = ld8(rp);
+    if (bias) bv = ld8(bias + n);
+  }
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float *pp = part + ((int64_t)p * M + m) * NP + n;
+  const int64_t step = (int64_t)PH * M * NP;
+  for (int k0 = 0; k0 < ksplit; k0 += 8) {
+    f32x4 q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      q[u] = k0 + u < ksplit ? *reinterpret_cast<const f32x4 *>(pp + (k0 + u) * step) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k0 + u < ksplit) v += q[u];
+  }
+  uint16_t *yp = y + (int64_t)b * s_yb + orow * s_yt + n;
+  if (VEC) {
+    if (bias) v += f32x4{h_lo(bv[0]), h_hi(bv[0]), h_lo(bv[1]), h_hi(bv[1])};
+    if (rp) v += f32x4{h_lo(rv[0]), h_hi(rv[0]), h_lo(rv[1]), h_hi(rv[1])};
+    u32x2 o = u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+    if (oa) o = snake4(o, oa + n, oib + n);
+    st8(yp, o);
+    return;
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     if (n + e >= Cout) continue;
     float o = v[e];
     if (bias) o += h_lo(bias[n + e]);
-    if (res) o += h_lo(res[(int64_t)b * s_rb + orow * s_rt + n + e]);
+    if (rp) o += h_lo(rp[e]);
     uint32_t ov = pack_f16x2(o, 0.f);
     if (oa) ov = snake2(ov, oa[n + e], oib[n + e], 0.f, 0.f);
-    y[(int64_t)b * s_yb + orow * s_yt + n + e] = (uint16_t)(ov & 0xffffu);
+    yp[e] = (uint16_t)(ov & 0xffffu);
   }
 }
 
@@ -584,7 +612,10 @@ static int launch_fin(const float *part, int64_t NP, int ksplit, const void *bia
                       int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, int64_t M, int TR, int Cout, int ph,
                       const float *oa, const float *oib, hipStream_t stream) {
   const int64_t threads = (int64_t)ph * M * ((Cout + 3) / 4);
-  hipLaunchKernelGGL(k_conv_fin, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, part, NP, ksplit,
+  const auto al8 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 7u) == 0; };
+  const bool vec = !(Cout & 3) && al8(bias) && al8(y) && !((s_yb | s_yt) & 3) &&
+                   (!res || (al8(res) && !((s_rb | s_rt) & 3)));
+  hipLaunchKernelGGL(vec ? k_conv_fin<true> : k_conv_fin<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, part, NP, ksplit,
                      (const uint16_t *)bias, (const uint16_t *)res, s_rb, s_rt, (uint16_t *)y, s_yb, s_yt, (int)M, TR,
                      Cout, ph, oa, oib);
   return (int)hipGetLastError();
