@@ -12,8 +12,8 @@
 //     point and the compiler's wait counts are exact (as loops, a unit's further steps drained every request in
 //     flight at the loop's head: 33.3 against 32.4 us per layer). Stores that only some lanes or waves make are
 //     buffer stores whose range check drops the others' (no branch around them either). 192 rows of 300..2048 keys:
-//     25.1 us per layer with every unit at the full row's 8 steps and the second unit g + G, 22.4 like this; all
-//     rows at 2048 keys 32.4 and 32.2; one row of 385 keys 6.0 and 5.5 (k_decode_unit).
+//     25.3 us per layer with every unit at the full row's 8 steps and the second unit g + G, 22.4 like this (all
+//     rows at 2048 keys: no difference); one row of 385 keys 6.0 and 5.5 (k_decode_unit).
 //   * Unit u starts at a step of its own (first_step; its waves take their tiles in the same rotated order). Units whose
 //     streams all start at the same offset and advance in step meet the same memory channels at the same
 //     time: a plain read of the peak-load bytes in this kernel's pattern took 35.2 us with every unit starting
@@ -21,7 +21,8 @@
 //   * Unit i + 1 is chosen and its metadata requested at unit i's second step, its inputs (q, or its qkv / bias /
 //     RoPE-table rows) at the third and, fused, rotated after the fourth, when they have long arrived. At the
 //     transition no wave waits for anything but its next tile. The lengths the choice needs are requested behind
-//     the first tiles (ahead of them, with the choice at the first step, all rows at 2048 keys took 32.5 us).
+//     the first tiles (ahead of them, with the choice at the first step, all rows at 2048 keys took 32.5 us
+//     against 32.2 in the same measurement).
 //   * The first unit's metadata and qkv / bias rows go out before any tile, its table rows as soon as the
 //     position returns and before the tiles, so q is ready about when the first tiles land.
 //   * A unit's k / v / q writes go out after its last step (at its first step, in the middle of the tile
@@ -74,15 +75,14 @@ __device__ __forceinline__ int steps_of(int keys, int least) {
   return max((n + 1) & ~1, least);
 }
 
-// The first step of a unit in workgroup g: one step on from a workgroup to the next, within a full row's steps (at
-// most 8, as far as the lengths of a 4096-position cache reach in ordinary use: with 16, every second workgroup
-// started at step 0 at 128..2048 keys, 14.1 us per layer at 64 rows against 13.05); step 0 where the unit has no
-// such step. The live tiles come in the same cyclic order whether n counts the full row's steps or only the unit's
-// own, so the sums are the same bits (the unfused launch requests its first tiles before it knows the length).
-__device__ __forceinline__ int first_step(int g, int cache_len, int n) {
-  const int nf = min(steps_of(cache_len, 2), 8);
-  int r = g & 7;
-  r = nf == 6 ? (r >= 6 ? r - 6 : r) : r & (nf - 1);
+// The first step of unit u = row * nkv + kh: one step on from a unit to the next, within the SPW steps the launch is
+// unrolled for; step 0 where the unit has no such step. It depends on the unit and its own length alone, so neither
+// the other rows' lengths nor the launch shape move a row's bits. The live tiles come in the same cyclic order
+// whether n counts the full row's steps or only the unit's own, so the sums are the same bits (the unfused launch
+// requests its first tiles before it knows the length). A 4096-position cache started within 8 of its 16 steps
+// instead: 192 rows of 4096 keys 61.7 us per layer against 60.1, of 128..2048 keys 21.9 against 22.1.
+__device__ __forceinline__ int first_step(int u, int spw, int n) {
+  const int r = u & (spw - 1);
   return r < n ? r : 0;
 }
 
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(64 * kRowsNW, 1) void k_decode_rows(
     un.crow = ok ? crow : -1;
     un.hi = (ok && exact) ? min(max(__builtin_amdgcn_readfirstlane(m.lraw), 0), cache_len) : 0;
     un.n = steps_of(exact ? un.hi : cache_len, least);
-    un.rot = first_step((int)blockIdx.x, cache_len, un.n);
+    un.rot = first_step(un.row * nkv + un.kh, SPW, un.n);
     const int64_t cb = (int64_t)(ok ? crow : 0) * s_kb + (int64_t)un.kh * s_kh;
     const uint32_t bound = ok ? (uint32_t)(exact ? un.hi : cache_len) * kRow : 0u;
     un.kr = make_rsrc_wave(kc + cb, bound);
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(64 * kRowsNW, 2) void k_decode_unit(
     vr = make_rsrc_wave(vc + cb, bound);
     if (first) {
       n = steps_of(exact ? hi : cache_len, 2);
-      rot = first_step(u, cache_len, n);
+      rot = first_step(u, SPW, n);
     }
   };
   // wave w: tiles w, w + NW, ... of the unit, starting at step rot (as k_decode_rows)

@@ -76,3 +76,38 @@ def test_fused_schedule(a8, dev, b, S, want):
     kind, shape = att.schedule(b, S, a8.ref_nsplit(b, NKV), fused=True)
     assert (kind, shape[2] if kind == "stream" else 0) == {"unit": ("stream", 2 * b), "pair": ("stream", b),
                                                            "split": ("split", 0)}[want]
+
+
+@pytest.mark.parametrize("b,S", [(12, 512), (67, 1500), (192, 2048), (33, 4096)])
+@pytest.mark.parametrize("fused", [True, False])
+def test_a_rows_bits_are_its_own(a8, dev, b, S, fused):
+    """A row's output depends on its own length alone: the same bits when every other row's length changes (and with
+    it the pairing by length), and the same bits with one unit a workgroup as with two."""
+    print(f"case: {b} rows x {S}, fused={fused}, kept rows among changed ones", flush=True)
+    g = torch.Generator().manual_seed(b + S)
+    kept = torch.arange(0, b, 3)
+    first = torch.randint(1, S + 1, (b,), generator=g, dtype=torch.int32)
+    qkv, bias = randn_bf16(g, b, W).to(dev), (torch.randn(W, generator=g) * 0.02).to(BF).to(dev)
+    kc, vc = randn_bf16(g, b, NKV, S, HD), randn_bf16(g, b, NKV, S, HD)
+    q0 = randn_bf16(g, b, NQ, HD).to(dev)
+    slot = torch.arange(b, dtype=torch.int32, device=dev)
+    cos, sin = a8.rope_tables(10000.0, HD, S, dev)
+    att = a8.DecodeAttention(max(16 * b, 64), NQ, NKV, HD, 16, dev)
+
+    def run(lens, per):
+        att.force_stream = (4, -(-S // 256), b if per == 2 else 2 * b)
+        k, v, out = kc.to(dev), vc.to(dev), torch.zeros(b, NQ, HD, dtype=BF, device=dev)
+        n = lens.to(dev)
+        if fused:
+            att.store_and_attend(qkv, bias, cos, sin, (n - 1), slot, torch.empty_like(q0), k, v, n, out)
+        else:
+            att(q0, k, v, n, out)
+        torch.cuda.synchronize()
+        return out.cpu().view(torch.int16)
+
+    want = run(first, 2)
+    assert torch.equal(run(first, 1), want)
+    for kind in range(3):
+        lens = torch.randint(1, S + 1, (b,), generator=g, dtype=torch.int32) if kind else torch.full_like(first, S)
+        lens[kept] = first[kept]
+        assert torch.equal(run(lens, 2)[kept], want[kept])
