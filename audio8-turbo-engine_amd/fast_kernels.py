@@ -258,20 +258,27 @@ class DecodeAttention:
             if (self.force_flat is not None or self.mode == "flat") and b <= self.FLAT_MAX_ROWS:
                 return "flat", self.flat_shape(b, cache_len)
             if self.mode == "auto":
-                if self._stream_pays(b, cache_len):
+                if self._stream_pays(b, cache_len, fused):
                     return "stream", self.stream_shape(b, cache_len)
                 if fused and 0 < cache_len <= self.SHORT_ROWS:
                     return "stream", self.short_rows_shape(b, cache_len)
         nsplit = max(1, min(int(nsplit), self.nsplit_max))
         return "split", self.launch_shape(b, cache_len, nsplit)
 
-    def _stream_pays(self, b: int, cache_len: int) -> bool:
-        """Mode "auto": the streaming schedule for many long rows (see the class docstring)."""
+    def _stream_pays(self, b: int, cache_len: int, fused: bool) -> bool:
+        """Mode "auto": the streaming schedule for many long rows (see the class docstring). Over more than 2048
+        positions an unfused call takes it from 3/4 of the compute units, a fused one from where
+        a8_decode_choose_stream does (5/8): the unfused launch requests its first tiles over the whole cache row, so
+        80 rows of 128..2048 keys in 4096 positions take it 18.4 us per layer against 14.4 for the split kernel,
+        where the fused launch, which has its row's length by then, takes 14.2 against 15.4. (64..4096 keys: fused
+        23.5 against 22.9.)"""
         if cache_len < 1024:
             return False
         nw, tpw, grid = self.stream_shape(b, cache_len)
         whole = nw * tpw * 64 >= cache_len
         units = b * self.nkv
+        if cache_len > 2048 and not fused and 4 * units < 3 * self.n_cu:
+            return False
         # two whole units per workgroup, or one per workgroup once the units reach half the compute units
         return whole and (units >= 2 * grid or (grid >= units and 2 * units >= self.n_cu))
 
