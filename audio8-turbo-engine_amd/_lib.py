@@ -75,6 +75,7 @@ SIGNATURES = {
 VOC_SIGNATURES = {
     "a8_conv_cl_snake": (_I, [_P, _L, _L, _P, _L, _L, _L, _I, _P, _P, _L, _L, _P, _L, _L, _P, _P, _P, _P,
                               _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P]),
+    "a8_conv_tile_query": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I, _L, _IP, _IP, _IP]),
 }
 
 _lock = threading.Lock()

@@ -33,6 +33,7 @@
 #include "../../include/a8voc.h"
 #include "conv_tile.h"
 #include "fp16_ops.h"
+#include <cmath>
 
 namespace a8 {
 
@@ -607,6 +608,27 @@ static ConvPlan conv_plan(int64_t M, int Cin, int Cout, int taps, int ph, bool a
   return pl;
 }
 
+// The plan that a workspace of ws_bytes allows.
+static ConvPlan conv_plan_for(int64_t M, int Cin, int Cout, int taps, int ph, int64_t ws_bytes) {
+  const ConvPlan pl = conv_plan(M, Cin, Cout, taps, ph);
+  return pl.ksplit > 1 && ws_bytes < pl.ws_bytes ? conv_plan(M, Cin, Cout, taps, ph, false) : pl;  // one pass
+}
+
+// The tile kernel's plan for a call that k_conv_cl would run as `pl` (with the same workspace): xkb 0 where k_conv_cl
+// takes it. One pass of k_conv_cl by its measured times (16 convs of 96 to 1536 channels, 12 to 224 steps of 32
+// channels, 20 to 65536 rows): 5.6 us and, a step, 0.18 us with one workgroup a compute unit, 0.33 (64 channels) or
+// 0.41 (96) with two. Against it the tile kernel in one pass, us: 768 channels k 7 on 192 / 384 / 576 workgroups 37.8 /
+// 55.8 / 82.9, tile 63.6 / 62.7 / 62.9; a stride-4 transposed conv to 192 channels on 192 / 512 / 576 workgroups 8.3 /
+// 15.1 / 19.6, tile 15.8 / 16.8 / 17.1. Beyond two a compute unit, or on 128-row tiles, the tile was always faster.
+static ConvTilePlan tile_plan(const ConvPlan &pl, int64_t M, int TR, int Tin, int Cin, int Cout, int taps, int dil,
+                              int ph, int64_t ws_bytes) {
+  double us = INFINITY;
+  const int64_t wgs = (M + 63) / 64 * pl.ntiles * ph;
+  if (pl.ksplit == 1 && (pl.WM == 1 || M <= 64) && wgs <= 512)
+    us = 5.6 + (double)(Cin / 32) * taps * (wgs <= 256 ? 0.18 : pl.NT <= 4 ? 0.33 : 0.41);
+  return conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, ph, false, ws_bytes, us);
+}
+
 // k_conv_fin over the partials of `ksplit` shares, rows of NP floats.
 static int launch_fin(const float *part, int64_t NP, int ksplit, const void *bias, const void *res, int64_t s_rb,
                       int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, int64_t M, int TR, int Cout, int ph,
@@ -658,16 +680,13 @@ extern "C" int a8_conv_cl_snake(const void *x, int64_t s_xb, int64_t s_xt, const
       s_wc < 0)
     return set_error(A8_EUNSUP, "conv_cl: x spans %lld bytes, w %lld (each must be below 2 GiB, strides >= 0)",
                      (long long)x_span, (long long)w_span);
-  ConvPlan pl = conv_plan(M, Cin, Cout, taps, ph);
-  if (pl.ksplit > 1 && (!ws || ws_bytes < pl.ws_bytes)) pl = conv_plan(M, Cin, Cout, taps, ph, false);  // one pass
+  const ConvPlan pl = conv_plan_for(M, Cin, Cout, taps, ph, ws ? ws_bytes : 0);
   if (pl.ksplit > 1 && !al16(ws)) return set_error(A8_EALIGN, "conv_cl: workspace must be 16-byte aligned");
   // the tile kernel where its preconditions hold: batch rows back to back, 16-byte stores, no snake on the load
   if (!snake_a && (B == 1 || s_xb == (int64_t)Tin * s_xt) && s_xt >= Cin && s_xt <= 65536 && al16(y) &&
       !((s_yb | s_yt) & 7) && (!res || (al16(res) && !((s_rb | s_rt) & 7))) &&
       !(reinterpret_cast<uintptr_t>(bias) & 7u)) {
-    ConvTilePlan tp = conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, ph, false, true);
-    if (tp.ksplit > 1 && (!ws || !al16(ws) || ws_bytes < tp.ws_bytes))
-      tp = conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, ph, false, false);
+    const ConvTilePlan tp = tile_plan(pl, M, TR, Tin, Cin, Cout, taps, dil, ph, ws && al16(ws) ? ws_bytes : 0);
     if (tp.xkb) {
       ConvTileArgs a{};
       a.x = (const uint16_t *)x, a.s_xt = s_xt, a.w = (const uint16_t *)w, a.s_wp = s_wp, a.s_wt = s_wt, a.s_wc = s_wc;
@@ -770,6 +789,23 @@ extern "C" int64_t a8_conv_cl_ws_bytes(int B, int TR, int Cin, int Cout, int tap
   return a > t ? a : t;
 }
 
+extern "C" int a8_conv_tile_query(int B, int Tin, int TR, int Cin, int Cout, int taps, int dil, int ph, int ru,
+                                  int64_t ws_bytes, int *mt_out, int *xkb_out, int *ksplit_out) {
+  using namespace a8;
+  if (B <= 0 || TR <= 0 || Cin <= 0 || Cout <= 0 || taps <= 0 || dil <= 0 || ph <= 0 || ws_bytes < 0 || !mt_out ||
+      !xkb_out || !ksplit_out || (int64_t)TR + (int64_t)(taps - 1) * dil > Tin || (int64_t)B * TR > INT32_MAX / 2)
+    return set_error(A8_EINVAL, "conv_tile_query: bad sizes B=%d Tin=%d TR=%d Cin=%d Cout=%d taps=%d dil=%d ph=%d", B,
+                     Tin, TR, Cin, Cout, taps, dil, ph);
+  const int64_t M = (int64_t)B * TR;
+  const ConvTilePlan tp = ru ? conv_tile_plan(M, TR, Tin, Cin, Cout, taps, dil, 1, true, 0, INFINITY)
+                             : tile_plan(conv_plan_for(M, Cin, Cout, taps, ph, ws_bytes), M, TR, Tin, Cin, Cout, taps,
+                                         dil, ph, ws_bytes);
+  *mt_out = tp.mt;
+  *xkb_out = tp.xkb;
+  *ksplit_out = tp.ksplit;
+  return 0;
+}
+
 extern "C" int a8_ru_cl(const void *xin, int64_t s_xb, int64_t s_xt, const void *w1, int64_t s_wt, int64_t s_wc,
                         const void *b1, const float *a2, const float *ib2, const void *w2, const void *b2,
                         const void *res, int64_t s_rb, int64_t s_rt, void *y, int64_t s_yb, int64_t s_yt, int B,
@@ -798,7 +834,7 @@ extern "C" int a8_ru_cl(const void *xin, int64_t s_xb, int64_t s_xt, const void 
                      (long long)w_span);
   if ((B == 1 || s_xb == (int64_t)Tin * s_xt) && s_xt >= C && s_xt <= 65536 && al16(y) && !((s_yb | s_yt) & 7) &&
       al16(res) && !((s_rb | s_rt) & 7) && !(reinterpret_cast<uintptr_t>(b2) & 7u)) {
-    const ConvTilePlan tp = conv_tile_plan(M, TR, Tin, C, C, taps, dil, 1, true, false);
+    const ConvTilePlan tp = conv_tile_plan(M, TR, Tin, C, C, taps, dil, 1, true, 0, INFINITY);
     if (tp.xkb) {
       ConvTileArgs a{};
       a.x = (const uint16_t *)xin, a.s_xt = s_xt, a.w = (const uint16_t *)w1, a.s_wt = s_wt, a.s_wc = s_wc;

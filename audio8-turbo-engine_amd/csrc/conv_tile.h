@@ -34,8 +34,11 @@ struct ConvTilePlan {
   bool narrow;
   int64_t ws_bytes;
 };
+// ws_bytes: what the caller's workspace holds (K is split no further); other_us: the time the launch would take on
+// k_conv_cl in one pass, infinite where that one would split K (its split never beat the tile's, however few shares
+// the workspace leaves the tile).
 ConvTilePlan conv_tile_plan(int64_t M, int TR, int Tin, int Cin, int Cout, int taps, int dil, int ph, bool ru,
-                            bool allow_split);
+                            int64_t ws_bytes, double other_us);
 // The split-K workspace conv_tile_plan would ask for, whatever the input rows.
 int64_t conv_tile_ws_bytes(int64_t M, int Cin, int Cout, int taps, int ph);
 int conv_tile_launch(const ConvTilePlan &pl, const ConvTileArgs &a, bool ru, hipStream_t stream);

@@ -362,13 +362,14 @@ static int64_t tile_count(int64_t M, int Cout, int ph, int mt) {
 // rows through every conv of the decoder, k = 1 .. 16): 6.5 us, the steps (one 32-channel slice of one tap) of a
 // share at the time a step takes with the compute unit's number of workgroups (mt 2: 0.40 us alone, 0.68 with a
 // second; mt 3: 0.56 and 1.05; further rounds in proportion), and for split K the finish: 4 us and 0.35 us per MB of
-// partials. It lies within 10 % of the measured times from 15 to 100 us; shares under 6 steps never paid.
-static int tile_split(int64_t M, int Cin, int Cout, int taps, int ph, int mt, bool allow_split, double *us) {
+// partials. It lies within 10 % of the measured times from 15 to 100 us; shares under 6 steps never paid. kmax: the
+// shares the caller's workspace holds.
+static int tile_split(int64_t M, int Cin, int Cout, int taps, int ph, int mt, int64_t kmax, double *us) {
   const int64_t tiles = tile_count(M, Cout, ph, mt), steps = (int64_t)(Cin / 32) * taps;
   const double mb = (double)ph * M * Cout * 4e-6;
   int best = 1;
-  const bool split = allow_split && steps >= 36 && (int64_t)ph * M * (Cout / 4) < ((int64_t)1 << 31);  // k_conv_fin
-  for (int k = 1; k <= (split ? 16 : 1); ++k) {
+  const bool split = steps >= 36 && (int64_t)ph * M * (Cout / 4) < ((int64_t)1 << 31);  // k_conv_fin
+  for (int k = 1; k <= (split ? 16 : 1) && (k == 1 || k <= kmax); ++k) {
     if (k > 1 && (k > Cin / 32 || steps / k < 6)) break;
     const int64_t n = (tiles * k + 255) / 256;
     const double step = mt == 2 ? (n == 1 ? 0.40 : n == 2 ? 0.68 : 0.36 * n) : n == 1 ? 0.56 : 0.53 * n;
@@ -383,14 +384,14 @@ int64_t conv_tile_ws_bytes(int64_t M, int Cin, int Cout, int taps, int ph) {
   int k = 1;
   double us;
   for (int mt = 2; mt <= 3; ++mt) {
-    const int km = tile_split(M, Cin, Cout, taps, ph, mt, true, &us);
+    const int km = tile_split(M, Cin, Cout, taps, ph, mt, 16, &us);
     k = km > k ? km : k;
   }
   return k > 1 ? (int64_t)k * ph * M * Cout * 4 : 0;
 }
 
 ConvTilePlan conv_tile_plan(int64_t M, int TR, int Tin, int Cin, int Cout, int taps, int dil, int ph, bool ru,
-                            bool allow_split) {
+                            int64_t ws_bytes, double other_us) {
   const ConvTilePlan none{0, 0, 1, false, 0};
   if (Cin % 32 || Cout % 96 || TR <= 0 || M <= 0 || (ru && Cout != 96 && Cout != 192)) return none;
   ConvTilePlan pl = none;
@@ -400,17 +401,19 @@ ConvTilePlan conv_tile_plan(int64_t M, int TR, int Tin, int Cin, int Cout, int t
     const int xkb = tile_xkb(TR, Tin, taps, dil, pl.narrow, ru, mt);
     if (!xkb) continue;
     double us;
-    const int k = tile_split(M, Cin, Cout, taps, ph, mt, allow_split && !ru, &us);
+    const int k = tile_split(M, Cin, Cout, taps, ph, mt, ru ? 1 : ws_bytes / (ph * M * Cout * 4), &us);
     if (!pl.mt || us < best) pl.mt = mt, pl.xkb = xkb, pl.ksplit = k, best = us;
   }
   if (!pl.mt) return none;
-  // Few tiles and a short K leave the chip idle: k_conv_cl's 64-row tiles are then faster (12 steps: 96 tiles of
-  // 128 x 192 take 11.7 us against 10.4, 192 tiles 12.5 against 13.5; 1x1, 12 steps: 96 tiles 12.7 against 12.0,
-  // 192 tiles 13.7 against 18.9; residual units of 192 and 96 channels: 128 tiles 28.9 against 26.0 and 19.2 against
-  // 15.7, 160 tiles 29.9 against 35.6 and 19.7 against 20.0). With >= 36 steps the split tile is faster at every size
-  // measured.
+  // Few tiles leave the chip idle. Split, that is in the model; in one pass k_conv_cl's 64-row tiles are then faster
+  // (its time: other_us), as they are with few tiles and nothing for the taps to share or little to do: 1x1 of 24, 12
+  // and 48 steps, 112 tiles 18.4 against 17.3, 12.9 against 12.0 and 29.9 against 28.6 us, 144 tiles 18.8 against
+  // 19.7, 13.2 against 13.8 and 30.4 against 33.2. Residual units of 192 and 96 channels: 128 tiles 28.9 against 26.0
+  // and 19.2 against 15.7, 160 tiles 29.9 against 35.6 and 19.7 against 20.0.
   const int64_t tiles = tile_count(M, Cout, ph, 2);
-  if (ru ? tiles < 160 : tiles < 128 && (int64_t)(Cin / 32) * taps < 36) return none;
+  if (ru ? tiles < 160
+         : best >= other_us || (pl.ksplit == 1 && tiles < 128 && (taps == 1 || (int64_t)(Cin / 32) * taps < 36)))
+    return none;
   if (pl.ksplit > 1) pl.ws_bytes = (int64_t)pl.ksplit * ph * M * Cout * 4;
   return pl;
 }

@@ -24,6 +24,15 @@ int a8_conv_cl_snake(const void *x, int64_t s_xb, int64_t s_xt, const void *w, i
                      const float *out_ib, int B, int Tin, int TR, int Cin, int Cout, int taps, int dil, int ph,
                      void *ws, int64_t ws_bytes, void *stream);
 
+/*
+ * a8_conv_tile_query: which instance of the tile kernel a8_conv_cl (ru = 0) or a8_ru_cl (ru = 1; Cin = Cout) takes for
+ * contiguous, aligned operands of these sizes, without a snake on the loads, and a workspace of ws_bytes: *mt the 32-row
+ * groups of a wave (2 or 3), *xkb the KiB of one slice of input rows, *ksplit the K shares; *mt = *xkb = 0 where the
+ * call runs on the general kernel. Host arithmetic, nothing is launched. For tests and tuning.
+ */
+int a8_conv_tile_query(int B, int Tin, int TR, int Cin, int Cout, int taps, int dil, int ph, int ru, int64_t ws_bytes,
+                       int *mt, int *xkb, int *ksplit);
+
 #ifdef __cplusplus
 }
 #endif

@@ -58,6 +58,26 @@ def test_conv_tile_edges(a8, dev, B, T, extra, Cin, Cout, taps, dil, ph, res, sp
     assert (got[:, 0] == 7.0).all() and (got[:, T * ph + 1] == 7.0).all()
 
 
+@pytest.mark.parametrize("shares", [0, 1, 2, 3, 4.5, 6])
+def test_conv_tile_workspace_sizes(a8, dev, shares):
+    """K shares as the workspace holds them, down to none (the general kernel then): nothing is written past it."""
+    from oracle import conv_ref as cref
+    M, Cin, Cout, taps = 250, 384, 384, 7
+    nws = int(shares * 4 * M * Cout)
+    print(f"case: conv_cl {M} rows, a workspace of {shares} shares", flush=True)
+    g = torch.Generator().manual_seed(77)
+    x = torch.randn(1, M + 6, Cin, generator=g).to(F16)
+    w = (torch.randn(1, taps, Cin, Cout, generator=g) / (taps * Cin) ** 0.5).to(F16)
+    bv = torch.randn(Cout, generator=g).to(F16)
+    want = cref.conv_cl(x, w, bv, M, taps, 1, 1, Cout)
+    ws = torch.full((nws + 4096,), 0x5a, dtype=torch.uint8, device=dev)
+    y = torch.empty(1, M, Cout, dtype=F16, device=dev)
+    a8.conv_cl(x.to(dev), w.to(dev), bv.to(dev), M, taps, 1, 1, y, ws=ws[:nws] if nws else None)
+    torch.cuda.synchronize()
+    assert _close(y, want)
+    assert (ws[nws:] == 0x5a).all()
+
+
 @pytest.mark.parametrize("B,T,C,dil", [(161, 128, 192, 9), (162, 127, 192, 1), (81, 515, 96, 9), (41, 1000, 96, 3)])
 def test_ru_tile_edges(a8, dev, B, T, C, dil):
     """The residual unit on the tile kernel (enough tiles for it): full and ragged tiles, both widths."""
