@@ -43,17 +43,17 @@ __device__ __forceinline__ rsrc_words_t rsrc_words(const void *base, uint32_t by
   return rsrc_words_t{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, 0x00020000u};
 }
 
-// bld16_lds as asm (see the head of the file). s_nop: the wait states a vector-written scalar operand and M0 need,
-// which the compiler does not add inside asm. (Nothing the compiler emits in these kernels uses M0.)
+// bld16_lds as asm (see the head of the file). M0 is an operand, so the compiler knows what the asm needs there and
+// sees to it again if it uses M0 itself. s_nop: the wait states a vector-written scalar operand and M0 need, which the
+// compiler does not add inside asm.
 __device__ __forceinline__ void dma16(rsrc_words_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
   lds = __builtin_amdgcn_readfirstlane(lds);  // (uniform; the compiler may have computed them in vector registers)
   soff = __builtin_amdgcn_readfirstlane(soff);
   asm volatile(
-      "s_mov_b32 m0, %0\n\t"
       "s_nop 4\n\t"
       "buffer_load_dwordx4 %1, %2, %3 offen lds"
       :
-      : "s"(lds), "v"(voff), "s"(r), "s"(soff)
+      : "{m0}"(lds), "v"(voff), "s"(r), "s"(soff)
       : "memory");
 }
 

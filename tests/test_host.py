@@ -145,3 +145,16 @@ def test_package_has_no_cpu_fallback():
                 src = re.sub(r"torch\.matmul\(x, w\.t\(\)(, out=y)?\)", "", src)
             for call in ("softmax(", "scaled_dot_product", "matmul(", "einsum(", "bmm(", ".exp("):
                 assert call not in src, (f, call)
+
+
+def test_asm_takes_m0_as_an_operand():
+    """M0 inside asm is an operand with that register as its constraint, never written by the asm's own text: the
+    compiler does not see the latter, and its own uses of M0 would go on with the wrong value."""
+    import os
+    import re
+    from conftest import ROOT
+    csrc = os.path.join(ROOT, "audio8-turbo-engine_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        with open(os.path.join(csrc, name)) as f:
+            code = "\n".join(line.split("//")[0] for line in f)
+        assert not re.search(r'"[^"\n]*\bm0\s*,', code), name
