@@ -28,6 +28,7 @@ import torch
 
 from .fast_kernels import conv_cl, conv_cl_ws_bytes, conv_out_tanh, ru_cl, snake_cat
 
+SNAKE_MAX_C = 1024  # the most channels of a conv with the snake on its loads (a8_conv_cl refuses more)
 F16 = torch.float16
 
 
@@ -213,10 +214,10 @@ class CLDecoder:
             for c1, c2, fu in units:
                 if fu is not None:
                     x = fu(x, b)
-                elif c2.state is None and c2.a is not None:
+                elif c2.state is None and c2.a is not None and c2.Cin <= SNAKE_MAX_C:
                     # c1's output feeds c2 alone, so c2's snake is applied as c1 stores it: once an element (c2's
                     # column tiles each applied it on their loads), and c2 runs on the tile kernel, which has no
-                    # snake on its loads
+                    # snake on its loads (wider units go on to c2's own check of them)
                     x = c2(c1(x, b, out_snake=(c2.a, c2.ib)), b, res=x, activated=True)
                 else:
                     x = c2(c1(x, b), b, res=x)

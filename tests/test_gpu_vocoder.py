@@ -136,3 +136,14 @@ def test_decoder_graph_replay_equals_eager(dev):
         ye = dec_e(x, B)
         torch.cuda.synchronize()
         assert torch.equal(yg, ye), f"frame {f}"
+
+
+def test_units_wider_than_the_load_snake_are_refused(dev):
+    """A two-conv unit of more channels than a conv takes with the snake on its loads is refused, as that conv is."""
+    say("case: CLDecoder 16->2064 ch, rate 2 (a unit of 1032 channels)")
+    voc = importlib.import_module("audio8-turbo-engine_amd.vocoder")
+    wts = voc.decoder_weights(cin=16, ch=2064, rates=(2,), k=3, dils=(1,), dev=dev, seed=1)
+    dec = voc.CLDecoder(wts, 1, dev)
+    with pytest.raises(NotImplementedError, match="snake on the load"):
+        dec(torch.randn(1, 2, 16, device=dev), 1)
+    torch.cuda.synchronize()
