@@ -4,9 +4,10 @@
 // arithmetic. One wave per (row, kv head) with nothing that a longer row needs (no ring, no next chunk, no merge): the
 // qkv and bias chunks, which depend on no metadata, and (without a row map) K and V are requested together with the
 // metadata, and only the table rows wait for the position; the streaming kernel asked for its 64-key tile first and
-// for the qkv chunks after the position. 192 rows x 10 positions in a graph: 5.9 -> 3.8 us per layer (a two-token pass
-// and 8 one-token passes of 4 layers 240 -> 171 us). Half a 64-key tile: the same operand layout, products and sum order as
-// compute_step's first 32 keys (the others would add zeros), so the same bits.
+// for the qkv chunks after the position. 192 rows x 10 positions in a graph: 5.9 -> 3.8 us per layer; a two-token pass
+// and 8 one-token passes of 4 layers 240 -> 169 us (171 with the last 64 bytes of the arguments left cold). Half a
+// 64-key tile: the same operand layout, products and sum order as compute_step's first 32 keys (the others would add
+// zeros), so the same bits.
 #pragma once
 #include "fused_qkv.h"
 
@@ -19,7 +20,7 @@ __global__ __launch_bounds__(64) void k_decode_short(uint16_t *kc, uint16_t *vc,
                                                      const int32_t *__restrict__ rowmap, uint16_t *__restrict__ out,
                                                      int64_t s_ob, int64_t s_oh, int b, int nq, int nkv, int group,
                                                      float sl2, StoreIn si) {
-  warm_kernargs<192>();  // the explicit arguments above span 0x00-0xd7
+  warm_kernargs<208>();  // the explicit arguments above span 0x00-0xcf
   __shared__ __attribute__((aligned(16))) uint16_t vt[kShortKeys * 64];
   const int lane = threadIdx.x, row = blockIdx.x / nkv, kh = blockIdx.x - row * nkv;
   TileLane tl;
