@@ -288,9 +288,12 @@ class DecodeAttention:
         self(q, kc, vc, lens, out, nsplit, rowmap=rowmap): the per-layer pair of fast_engine.py:127-132 with
         the store done by the decode's own kernel (a8_store_decode_stream / _split / _flat, whichever
         schedule the call takes): one launch, or two with the split schedule's combine.
-        Same results bit for bit, given that no row attends a cache row another row stores into: the
-        engine's decode tick (slot[r] = r, rowmap None, fast_engine.py:752-753) or distinct slots with
-        rowmap = slot. Rows sharing a slot, like the fast stack's 2-token first pass, need the two calls.
+        Same results bit for bit as the two calls at this call's launch shape, given that no row attends a
+        cache row another row stores into (mode "auto" may give the two calls another shape, see schedule():
+        over short rows, and for some row counts over more than 2048 positions; they then sum the keys in
+        another order): the engine's decode tick (slot[r] = r, rowmap None, fast_engine.py:752-753) or
+        distinct slots with rowmap = slot. Rows sharing a slot, like the fast stack's 2-token first pass,
+        need the two calls.
         The rotated q is an intermediate of the pair that the engine never reads back: with write_q=False
         it is not written (a saving of ~1 us per layer at the peak load). One difference where the
         reference is undefined: a row whose position lies outside the RoPE tables attends with q = 0 here

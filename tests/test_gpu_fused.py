@@ -160,9 +160,9 @@ def test_attn_stack_tick_fused_matches_unfused(a8, dev):
         assert _bits_equal(st[0].kc[i], st[1].kc[i]) and _bits_equal(st[0].vc[i], st[1].vc[i])
 
 
-@pytest.mark.parametrize("b,S", [(1, 512), (192, 10), (64, 300), (5, 65)])
+@pytest.mark.parametrize("b,S", [(1, 512), (192, 10), (64, 300), (5, 65), (3, 513), (20, 1000), (7, 1024)])
 def test_store_and_attend_short_rows_auto(a8, ref, dev, b, S):
-    """Mode "auto" runs a fused call over short rows (cache_len <= 512) as one streaming launch with one
+    """Mode "auto" runs a fused call over short rows (cache_len <= 1024) as one streaming launch with one
     workgroup per (row, kv head): the same bits as the two calls at that launch shape, and the oracle's
     answer (the engine's tick: slot = row, no row map)."""
     say(f"case: fused short rows auto, b={b} S={S}")
