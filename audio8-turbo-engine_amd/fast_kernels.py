@@ -161,7 +161,8 @@ class DecodeAttention:
         launch pays its memory round trips while the KV stream fills the queues).
       mode "auto" (default): "stream" when the rows are whole units (row, kv head) of 1024+ keys that
         either give every workgroup of the grid two of them -- the peak-load shape -- or, one per
-        workgroup, number at least half the compute units (tick buckets of 64-128 slots at KV 2048); for
+        workgroup, number at least half the compute units (tick buckets of 64-128 slots at KV 2048; over
+        more than 2048 positions 5/8 of them, 3/4 in an unfused call); for
         the fused store + decode (store_and_attend) also when rows are short (cache_len <= 1024: one
         workgroup per (row, kv head) holds the whole row, so the store, the decode and the merge take
         one launch); else "split"."""
@@ -236,9 +237,12 @@ class DecodeAttention:
         self._shapes[key] = (grid.value,)
         return self._shapes[key]
 
-    # fused calls: rows of at most this many cache positions take one workgroup each. At 1024 positions (lengths up to
-    # the cache) one launch took 4.8 / 7.4 / 7.9 us at 1 / 8 / 32 rows against 8.1 / 8.9 / 9.6 for split + combine; at
-    # 2048 the long rows turn it round (16 rows of up to 1400 keys: 9.4 against 8.9)
+    # fused calls: rows of at most this many cache positions take one workgroup each. At 520 to 1024 positions, 1 to 400
+    # rows, lengths full, spread up to the cache or to a quarter of it, one launch was never slower than split + combine
+    # (1024 positions, spread: 4.8 / 8.4 / 10.5 / 16.4 / 26.0 us at 1 / 32 / 128 / 192 / 400 rows against 8.2 / 9.3 /
+    # 11.6 / 17.5 / 28.3). Two units a workgroup are faster for more than 128 full rows only (1000 positions, 160 rows:
+    # 17.9 against 20.8 full, but 14.8 against 14.0 spread and 11.8 against 10.2 short). At 2048 positions the long rows
+    # turn it round (16 rows of up to 1400 keys: 9.4 against 8.9)
     SHORT_ROWS = 1024
 
     def short_rows_shape(self, b: int, cache_len: int):
