@@ -968,7 +968,8 @@ def conv_cl(xin, w, bias, TR, taps, dil, ph, out, res=None, f16acc=True, cfg=Non
     of [Cout], to the stored fp16 outputs (the bits the next conv would read with it as its `snake`). Accumulation
     is fp32 (f16acc, the reference's fp16 slice sums, and cfg, its Triton tile choice, are accepted and
     unused). ws: an optional device byte buffer the launch may use to split K on short inputs (its size:
-    conv_cl_ws_bytes); without one, or when it is too small, K is not split. Nothing is allocated here."""
+    conv_cl_ws_bytes); without one K is not split, in a smaller one it may be split less. Nothing is allocated
+    here."""
     for name, t, d in (("xin", xin, 3), ("w", w, 4), ("out", out, 3)):
         _need(isinstance(t, torch.Tensor) and t.dtype == _F16, f"{name} must be a float16 tensor", TypeError)
         _need(t.dim() == d and t.stride(-1) == 1, f"{name} must have {d} dims with a contiguous last dim")

@@ -57,8 +57,8 @@ class CLConv:
     (_CLConv, fast_engine.py:178-233). weight / bias are the module's tensors; alpha the snake's [Cin] (or
     None); dilation for a Conv1d, stride for a ConvTranspose1d (trans=True). tmax: the most input rows a call
     takes (a frame's length at this conv); the split-K workspace is sized once for every row count up to Bmax
-    at tmax rows. A call with more rows or a shape needing more runs K unsplit (nothing is allocated in a
-    call)."""
+    at tmax rows. A call with more rows or a shape needing more splits K less or not at all (nothing is
+    allocated in a call)."""
 
     def __init__(self, weight, bias, Bmax, dev, states, alpha=None, trans=False, stride=1, dilation=1, tmax=None):
         self.W, self.taps, self.ph = pack_conv(weight.to(dev), trans, stride)

@@ -415,8 +415,9 @@ int a8_gemm_small_norm_pf(const void *x, int64_t ldx, const void *w, int64_t ldw
  *   wider inputs take snake_cat first). fp32 accumulation.
  *   ws / ws_bytes: an optional 16-byte aligned device workspace; with a8_conv_cl_ws_bytes(...) bytes the
  *   kernel may split K across workgroups (fixed-order fp32 sums: the same result with or without it).
- * a8_conv_cl_ws_bytes: the workspace a8_conv_cl would use for these sizes (0: none). No counterpart in the
- *   reference (its Triton conv splits nothing); lets the caller allocate from its own pool.
+ * a8_conv_cl_ws_bytes: the workspace a8_conv_cl would use for these sizes (0: none; in a smaller one K is split
+ *   less, or not). No counterpart in the reference (its Triton conv splits nothing); lets the caller allocate from
+ *   its own pool.
  * a8_snake_cat replaces serve/fast_kernels.py:718-729 (snake_cat, kernel 695-715):
  *   y[b] = concat(state[b] (CTX rows), snake(x[b]) (T rows)), C a multiple of 8; a / ib NULL: no snake.
  */
